@@ -29,7 +29,8 @@ SYMBOLS = (
     "sas_target_units", "sas_plan", "sas_forward", "sas_resolve", "sas_attend", "sas_combine",
     "sas_debug_rows", "sas_graph_capture", "sas_graph_launch", "sas_graph_destroy",
     "sas_metadata_legacy", "sas_forward_noalloc", "sas_attend_timed",
-    "sas_backward_workspace_size", "sas_backward", "sas_debug_lists",
+    "sas_backward_workspace_size",
+    "sas_backward_workspace_size_for", "sas_backward", "sas_debug_lists",
 )
 SAS_SCRATCH_BYTES = 160 << 20  # include/sas.h: the fixed workspace of sas_forward_noalloc
 
@@ -110,6 +111,7 @@ def load():
         lib.sas_forward_noalloc.argtypes = [PP, PT, P, P, P]
         lib.sas_attend_timed.argtypes = [PP, PT, P, P, S, P, P, P, P]
         lib.sas_backward_workspace_size.argtypes = [PP, ctypes.POINTER(S)]
+        lib.sas_backward_workspace_size_for.argtypes = [PP, I, ctypes.POINTER(S)]
         lib.sas_backward.argtypes = [PP, PT, P, P, P, P, P, P, P, P, S, P]
         lib.sas_graph_capture.argtypes = [PP, PT, P, P, S, P, ctypes.POINTER(P)]
         lib.sas_graph_launch.argtypes = [P, P]

@@ -186,8 +186,8 @@ class SasLaunch:
         T, H = p.total_tokens, p.num_heads_q
         dev = self.device
         need = ctypes.c_size_t()
-        _lib.check(lib.sas_backward_workspace_size(ctypes.byref(p), ctypes.byref(need)),
-                   "sas_backward_workspace_size")
+        _lib.check(lib.sas_backward_workspace_size_for(ctypes.byref(p), int(kv_grad), ctypes.byref(need)),
+                   "sas_backward_workspace_size_for")
 
         def pool_grad(pool):
             n = 1 + sum((d - 1) * st for d, st in zip(pool.shape, pool.stride()))

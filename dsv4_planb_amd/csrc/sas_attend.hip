@@ -1273,7 +1273,7 @@ __global__ __launch_bounds__(256, 1) void attend_kernel(
     const bool last = split < 0 || split == tk[TK_SPLITS] - 1;
     own_hi = last ? a.list_stride : min(ur[2], a.list_stride);
     int nwin = 0;
-    const int nc = resolve_rows(a, tk, true, t, ur[1], own_hi,
+    const int nc = resolve_rows<false>(a, tk, true, t, ur[1], own_hi,
                                 *reinterpret_cast<RsShared*>(sm.tiles), rs, nwin);
     live = make_int2(nwin, nwin < 0 ? 0 : nc);
     if (rs.tok && threadIdx.x == 0 && last) rs.tok[t] = live;

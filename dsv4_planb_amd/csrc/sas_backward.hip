@@ -85,11 +85,16 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(SasFwdArgs a, int dqk,
                                                        const float* __restrict__ sinks,
                                                        float* __restrict__ dterm,
                                                        float* __restrict__ sterm,
-                                                       float* __restrict__ dq) {
+                                                       float* __restrict__ dq,
+                                                       int* __restrict__ flags) {
   constexpr int DV = 512;
   const int HB = (a.H + 3) / 4;
   const int t = blockIdx.x / HB, h = (blockIdx.x - t * HB) * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
+  if (flags && threadIdx.x == 0 && blockIdx.x == t * HB) {
+    flags[1 + t] = 0;
+    if (t == 0) flags[0] = 0;
+  }
   if (h >= a.H) return;
   const bool ok = plan_matches(plan, a);
   const int* tk = plan + SAS_PLAN_HDR + (size_t)t * SAS_TOK_W;
@@ -126,7 +131,20 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(SasFwdArgs a, int dqk,
   }
 }
 
-template <int DQK, int QT>
+// The spill (see SasBwdLayout): record 0 is all zeros, then record 1 + (t - t0) stride
+// + p for list position p of token t; a record is, per 32-head chunk, 64 B of
+// scale dS and 64 B of P in the query dtype.  flags[0] counts and flags[1 + t] marks
+// the tokens with an infinity or a NaN in q or dO: the tile kernel, whose masked rows
+// multiply a token's q and dO by zeros, leaves those to the per-unit kernel.
+struct SasBwdSpill {
+  int t0, t1;      // tokens of this run
+  int stride;      // list positions per token
+  int row_bytes;
+  uint8_t* data;
+  int* flags;
+};
+
+template <int DQK, int QT, bool SPILL>
 __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint16_t* __restrict__ q,
                                                         const uint16_t* __restrict__ dout,
                                                         const uint64_t* __restrict__ addr_list,
@@ -134,7 +152,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
                                                         const float* __restrict__ lse,
                                                         const float* __restrict__ dterm,
                                                         const int* __restrict__ plan,
-                                                        float* __restrict__ dq) {
+                                                        float* __restrict__ dq, SasBwdSpill sp) {
   constexpr int DV = 512;
   constexpr int KS = DQK / 32;         // k-steps of S^T = K Q^T (18 / 16)
   constexpr int VKS = DV / 32;         // k-steps of dP^T = V dO^T (16)
@@ -145,12 +163,15 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
   // two tiles: the one computed on and the next one, stored from registers after
   // the MFMAs of this one
   __shared__ __attribute__((aligned(16))) uint8_t kt[2][BW_TILE * KSTR];
+  // SPILL: a wave's P and dS of a tile, [16 heads][32 keys] each, for the transpose
+  __shared__ __attribute__((aligned(16))) uint8_t tp[SPILL ? 4 * 2048 : 16];
 
   const int HG = (a.H + BW_HEADS - 1) / BW_HEADS;
   const int u = blockIdx.x / HG, hg = blockIdx.x - u * HG;
   if (!plan_matches(plan, a) || u >= plan[PH_UNITS]) return;  // refused plan: prep zeroed dq
   const int* ur = plan + SAS_PLAN_HDR + (size_t)SAS_TOK_W * a.T + (size_t)u * SAS_UNIT_W;
   const int t = ur[0], split = ur[3];
+  if (SPILL && (t < sp.t0 || t >= sp.t1)) return;  // a token of another run
   if (split < 0) return;  // a q row no batch owns: zero (bwd_prep_kernel)
   const int* tk = plan + SAS_PLAN_HDR + (size_t)t * SAS_TOK_W;
   const int splits = tk[TK_SPLITS];
@@ -212,6 +233,37 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
   }
   const float lse2 = lse[th] * LOG2E, dh = dterm[th];
   const float c = a.scale_log2;
+  const float scale = c * 0.6931471805599453f;
+  if constexpr (SPILL) {
+    // an infinity or a NaN: all exponent bits set (both halves of each dword)
+    constexpr uint32_t EXP = QT == 0 ? 0x7f80u : 0x7c00u;
+    bool bad = false;
+    auto check = [&](const u32x4_t& v) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        bad = bad || (v[e] & EXP) == EXP || ((v[e] >> 16) & EXP) == EXP;
+    };
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) check(qf[ks]);
+#pragma unroll
+    for (int ks = 0; ks < VKS; ++ks) check(of[ks]);
+    if (__any(bad) && lane == 0) {
+      sp.flags[1 + t] = 1;
+      atomicAdd(sp.flags, 1);
+    }
+  }
+  // SPILL: the wave's P and dS go through LDS: lane (n16, g) writes its 8 keys of head
+  // n16 (16 B: positions 8 g .. + 7 of the head's 64-B row, key 16 kb + 4 g + r at
+  // position 8 g + 4 kb + r), and ds_read_b64_tr_b16 returns 4 heads (4 g .. + 3) of
+  // one position per lane, stored as 8 B of its key's record.  The 32-B halves of a row
+  // are swapped for heads 4 .. 7 and 12 .. 15, so that the transposed reads touch every
+  // bank once per 256 B.
+  uint8_t* const tpw = tp + (SPILL ? w * 2048 : 0);
+  const bool sp_wave = SPILL && hg * BW_HEADS + w * 16 < sp.row_bytes / 4;  // a padded head chunk ends
+  uint8_t* sp_row = nullptr;
+  if constexpr (SPILL)
+    sp_row = sp.data + (1 + (size_t)(t - sp.t0) * sp.stride) * sp.row_bytes +
+             (2 * hg + (w >> 1)) * 128 + (16 * (w & 1) + 4 * g) * 2;
   bw_f32x4 acc[NDB];
 #pragma unroll
   for (int i = 0; i < NDB; ++i) acc[i] = bw_f32x4{0.f, 0.f, 0.f, 0.f};
@@ -254,18 +306,50 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
       }
     }
     // P = e^(s - lse) and dS = P (dP - D) for keys 16 kb + 4 g + r of head n16
-    float ds[8];
+    float ds[8], pr[8];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const bool valid = rb + 16 * kb + 4 * g + r < r1;
         const float p = valid ? exp2f(fmaf(s[kb][r], c, -lse2)) : 0.f;
+        pr[4 * kb + r] = p;
         ds[4 * kb + r] = p * (dp[kb][r] - dh);
       }
     u32x4_t bds;
 #pragma unroll
     for (int e = 0; e < 4; ++e) bds[e] = pack2_q16<QT>(ds[2 * e], ds[2 * e + 1]);
+    if constexpr (SPILL) {
+      if (sp_wave) {
+        u32x4_t xs, xp;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {  // (heads at or past H: zeros)
+          xs[e] = hvalid ? pack2_q16<QT>(ds[2 * e] * scale, ds[2 * e + 1] * scale) : 0u;
+          xp[e] = hvalid ? pack2_q16<QT>(pr[2 * e], pr[2 * e + 1]) : 0u;
+        }
+        const int wo = 64 * n16 + 16 * (g ^ (2 * ((n16 >> 2) & 1)));
+        *reinterpret_cast<u32x4_t*>(tpw + wo) = xs;
+        *reinterpret_cast<u32x4_t*>(tpw + 1024 + wo) = xp;
+        const uint8_t* ro = tpw + 64 * (4 * g + (n16 >> 2)) + 8 * (n16 & 3);
+        tr_s4 v[2][2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int z = 0; z < 2; ++z)
+            v[x][z] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) tr_s4*)(ro + 1024 * z + 32 * (x ^ (g & 1))));
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          const int p = rb + 16 * ((n16 >> 2) & 1) + 4 * (2 * x + (n16 >> 3)) + (n16 & 3);
+          if (p < r1 && p < sp.stride) {
+            typedef __attribute__((address_space(1))) tr_s4 g_s4;
+            uint8_t* dst = sp_row + (size_t)p * sp.row_bytes;
+            *(g_s4*)(uintptr_t)dst = v[x][0];
+            *(g_s4*)(uintptr_t)(dst + 64) = v[x][1];
+          }
+        }
+      }
+    }
     // dq^T += K^T dS^T.  A = dimensions 16 db + n16 of keys 4 g .. 4 g + 3 (then 16 +
     // 4 g ..), read transposed from the row-major tile: within each 16-lane block,
     // ds_read_b64_tr_b16 gives lane j element j & 3 of the 8 bytes lane (j >> 2) + 4 e
@@ -300,7 +384,6 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
   }
   if (!hvalid) return;
   // lane holds dimensions 16 db + 4 g .. + 3 of head h
-  const float scale = c * 0.6931471805599453f;
   float* dqr = dq + ((size_t)t * a.H + h) * DQK + 4 * g;
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
@@ -344,29 +427,41 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
 // ---------------------------------------------------------------------------
 constexpr int DK_HEADS = 32;  // heads per group
 
+//
+// tiles (the rows bwd_dkv_tile_kernel takes): 0 none, 1 the window rows, 2 all; then
+// flags marks the tokens whose rows all stay here.
 template <int DQK, int QT>
-__global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(
-    SasFwdArgs a, const uint16_t* __restrict__ q, const uint16_t* __restrict__ dout,
-    const uint64_t* __restrict__ addr_list, const int* __restrict__ row_codes,
-    const int2* __restrict__ tok, const float* __restrict__ lse, const float* __restrict__ dterm,
-    const int* __restrict__ plan, float* __restrict__ d_ori, float* __restrict__ d_cmp) {
+struct DkvLds {
+  static constexpr int KSTR = DQK * 2 + 16;      // row-major K tile and staged q: row stride in bytes
+  static constexpr int OSTR = 512 * 2 + 16;      // staged dO: row stride in bytes
+  static constexpr int TS = 2 * DK_HEADS + 16;   // [key][head] rows of dS^T and P^T: bytes per key
+  __attribute__((aligned(16))) uint8_t kt[BW_TILE * KSTR];
+  __attribute__((aligned(16))) uint8_t qs[DK_HEADS * KSTR];
+  __attribute__((aligned(16))) uint8_t os[DK_HEADS * OSTR];
+  __attribute__((aligned(16))) uint8_t dst[BW_TILE * TS];
+  __attribute__((aligned(16))) uint8_t ptr[BW_TILE * TS];
+};
+
+template <int DQK, int QT>
+__device__ __forceinline__ void dkv_unit(
+    int u, DkvLds<DQK, QT>& sm, const SasFwdArgs& a, const uint16_t* __restrict__ q,
+    const uint16_t* __restrict__ dout, const uint64_t* __restrict__ addr_list,
+    const int* __restrict__ row_codes, const int2* __restrict__ tok, const float* __restrict__ lse,
+    const float* __restrict__ dterm, const int* __restrict__ plan, float* __restrict__ d_ori,
+    float* __restrict__ d_cmp, int tiles, const int* __restrict__ flags) {
   constexpr int DV = 512;
   constexpr int KS = DQK / 32;         // k-steps of S^T = K Q^T (18 / 16)
   constexpr int VKS = DV / 32;         // k-steps of dP^T = V dO^T (16)
   constexpr int NDB = DQK / 16;        // 16-dimension blocks of G (36 / 32)
   constexpr int CH = DQK / 8;          // 16-B chunks per row of K or q
   constexpr int CHO = DV / 8;          // 16-B chunks per row of dO
-  constexpr int KSTR = DQK * 2 + 16;   // row-major K tile and staged q: row stride in bytes
-  constexpr int OSTR = DV * 2 + 16;    // staged dO: row stride in bytes
-  constexpr int TS = 2 * DK_HEADS + 16;  // [key][head] rows of dS^T and P^T: bytes per key
-  __shared__ __attribute__((aligned(16))) uint8_t kt[BW_TILE * KSTR];
-  __shared__ __attribute__((aligned(16))) uint8_t qs[DK_HEADS * KSTR];
-  __shared__ __attribute__((aligned(16))) uint8_t os[DK_HEADS * OSTR];
-  __shared__ __attribute__((aligned(16))) uint8_t dst[BW_TILE * TS];
-  __shared__ __attribute__((aligned(16))) uint8_t ptr[BW_TILE * TS];
+  constexpr int KSTR = DkvLds<DQK, QT>::KSTR, OSTR = DkvLds<DQK, QT>::OSTR, TS = DkvLds<DQK, QT>::TS;
+  uint8_t* const kt = sm.kt;
+  uint8_t* const qs = sm.qs;
+  uint8_t* const os = sm.os;
+  uint8_t* const dst = sm.dst;
+  uint8_t* const ptr = sm.ptr;
 
-  const int u = blockIdx.x;
-  if (!plan_matches(plan, a) || u >= plan[PH_UNITS]) return;
   const int* ur = plan + SAS_PLAN_HDR + (size_t)SAS_TOK_W * a.T + (size_t)u * SAS_UNIT_W;
   const int t = ur[0], split = ur[3];
   if (split < 0) return;  // a q row no batch owns: it reads no rows
@@ -374,7 +469,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(
   const int2 tr = tok[t];  // row counts at the call's lengths (the resolver's)
   if (tr.x < 0) return;    // refused token: it reads no rows
   const int nwin = tr.x;   // list positions below it are window rows (raw pool)
-  const int r0 = ur[1];
+  int r0 = ur[1];
+  if (tiles && !flags[1 + t]) {  // the window rows, or all, are bwd_dkv_tile_kernel's
+    if (tiles == 2) return;
+    r0 = max(r0, nwin);
+  }
   const int r1 = min(ur[3] == tk[TK_SPLITS] - 1 ? tr.x + tr.y : min(ur[2], tr.x + tr.y),
                      a.list_stride);
   const int ntiles = r1 > r0 ? (r1 - r0 + BW_TILE - 1) / BW_TILE : 0;
@@ -596,6 +695,26 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(
       for (int r = 0; r < 4; ++r)
         if (rowp[r]) gatomic_add(rowp[r] + dim, gacc[k][r]);
     }
+  }
+}
+
+// Workgroup x takes units x, x + gridDim, ...  Where the tiles take every row
+// (tiles == 2), one look at the count of marked tokens ends it.
+template <int DQK, int QT>
+__global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(
+    SasFwdArgs a, const uint16_t* __restrict__ q, const uint16_t* __restrict__ dout,
+    const uint64_t* __restrict__ addr_list, const int* __restrict__ row_codes,
+    const int2* __restrict__ tok, const float* __restrict__ lse, const float* __restrict__ dterm,
+    const int* __restrict__ plan, float* __restrict__ d_ori, float* __restrict__ d_cmp, int tiles,
+    const int* __restrict__ flags) {
+  __shared__ DkvLds<DQK, QT> sm;
+  if (tiles == 2 && flags[0] == 0) return;
+  if (!plan_matches(plan, a)) return;
+  const int units = plan[PH_UNITS];
+  for (int u = blockIdx.x; u < units; u += gridDim.x) {
+    dkv_unit<DQK, QT>(u, sm, a, q, dout, addr_list, row_codes, tok, lse, dterm, plan, d_ori, d_cmp,
+                      tiles, flags);
+    __syncthreads();  // every wave is done with the unit's LDS
   }
 }
 

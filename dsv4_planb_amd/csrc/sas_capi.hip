@@ -17,6 +17,7 @@
 #include "sas_kernels.hip"
 #include "sas_attend.hip"
 #include "sas_backward.hip"
+#include "sas_backward_tile.hip"
 
 namespace {
 
@@ -150,6 +151,8 @@ sas::SasResolveArgs resolve_args(const sas_params_t* p, const sas_tensors_t* t, 
   r.ori_scale = t->ori_kv_scale;
   r.cmp_scale = t->cmp_kv_scale;
   r.scale = w.scale;
+  r.inv = nullptr;
+  r.inv_rows = 0;
   return r;
 }
 
@@ -211,9 +214,10 @@ int launch_attend(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
 }
 
 // The resolver stage; codes: also write the row codes (the forward reads addresses
-// only; the backward and sas_debug_rows read the codes).
+// only; the backward and sas_debug_rows read the codes).  inv: also the inverse lists.
 int resolve_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
-                  size_t ws_bytes, sas_stream_t stream, bool codes) {
+                  size_t ws_bytes, sas_stream_t stream, bool codes, uint32_t* inv = nullptr,
+                  int inv_rows = 0) {
   int rc = sas_validate(p);
   if (rc) return rc;
   if ((rc = check_tensors(p, t))) return rc;
@@ -224,7 +228,9 @@ int resolve_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
   if (p->total_tokens == 0) return SAS_OK;
   sas::SasResolveArgs r = resolve_args(p, t, w);
   if (!codes) r.rows = nullptr;
-  hipLaunchKernelGGL(sas::resolve_kernel, dim3(p->total_tokens), dim3(sas::RS_NT), 0,
+  r.inv = inv;
+  r.inv_rows = inv_rows;
+  hipLaunchKernelGGL(inv ? &sas::resolve_kernel<true> : &sas::resolve_kernel<false>, dim3(p->total_tokens), dim3(sas::RS_NT), 0,
                      (hipStream_t)stream, fwd_args(p, target), plan, r);
   return launch_status();
 }
@@ -279,6 +285,16 @@ int forward_impl(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
     if ((rc = launch_attend(p, t, plan, w, target, stream, nullptr, nullptr, false))) return rc;
   }
   return combine_stage(p, t, plan, ws, ws_bytes, stream, status_out);
+}
+
+int bwd_layout(const sas_params_t* p, SasBwdLayout* L) {
+  size_t fwd = 0;
+  const int rc = sas_workspace_size(p, &fwd);
+  if (rc) return rc;
+  const int64_t cmp_cap = p->scenario >= 2 ? (int64_t)p->cmp_table_len * p->cmp_block_size : 0;
+  *L = sas_bwd_layout(fwd, p->total_tokens, p->batch, p->num_heads_q, p->scenario, p->ori_win_left,
+                      list_k(p), cmp_cap);
+  return SAS_OK;
 }
 
 }  // namespace
@@ -424,13 +440,16 @@ int sas_forward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* pl
 }
 
 int sas_backward_workspace_size(const sas_params_t* p, size_t* bytes) {
+  return sas_backward_workspace_size_for(p, 1, bytes);
+}
+
+int sas_backward_workspace_size_for(const sas_params_t* p, int kv_grad, size_t* bytes) {
   int rc = sas_validate(p);
   if (rc) return rc;
   if (!bytes) return SAS_ERR_NULL;
-  size_t fwd = 0;
-  if ((rc = sas_workspace_size(p, &fwd))) return rc;
-  const size_t th = (size_t)(p->total_tokens > 0 ? p->total_tokens : 1) * p->num_heads_q;
-  *bytes = fwd + 2 * sas_align256(th * 4);  // D and the sink term per (token, head)
+  SasBwdLayout L;
+  if ((rc = bwd_layout(p, &L))) return rc;
+  *bytes = kv_grad ? L.total : L.base_total;
   return SAS_OK;
 }
 
@@ -443,19 +462,18 @@ int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
   if (!dout || !dq || !dsinks || !t->lse) return SAS_ERR_NULL;
   if (p->kv_dtype == SAS_DT_FP8E4M3) return SAS_ERR_NOT_IMPLEMENTED;
   if (!aligned16(dout) || !aligned16(dq)) return SAS_ERR_SHAPE;
-  size_t need = 0;
-  if ((rc = sas_backward_workspace_size(p, &need))) return rc;
-  if (!ws || ws_bytes < need) return SAS_ERR_WORKSPACE;
+  const bool kv_grad = d_ori_kv || d_cmp_kv;
+  SasBwdLayout L;
+  if ((rc = bwd_layout(p, &L))) return rc;
+  if (!ws || ws_bytes < (kv_grad ? L.total : L.base_total)) return SAS_ERR_WORKSPACE;
   const int target = target_units(p);
   Ws w;
   if ((rc = carve(p, ws, ws_bytes, target, &w))) return rc;
   hipStream_t s = (hipStream_t)stream;
   const int T = p->total_tokens, H = p->num_heads_q;
-  const SasWsLayout W = sas_ws_layout(T, list_k(p), H, p->head_dim_v, target, p->scenario,
-                                      p->ori_win_left, false);
-  float* dterm = reinterpret_cast<float*>(static_cast<char*>(ws) + W.total);
-  float* sterm = reinterpret_cast<float*>(static_cast<char*>(ws) + W.total +
-                                          sas_align256((size_t)T * H * 4));
+  char* base = static_cast<char*>(ws);
+  float* dterm = reinterpret_cast<float*>(base + L.off_dterm);
+  float* sterm = reinterpret_cast<float*>(base + L.off_sterm);
   if (T == 0) {  // no tokens: dsinks = 0 (a kernel, not a memset, so the call can be captured)
     hipLaunchKernelGGL(sas::bwd_dsink_kernel, dim3(H), dim3(256), 0, s, 0, H,
                        static_cast<const float*>(sterm), dsinks);
@@ -467,43 +485,83 @@ int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
     if ((rc = launch_status())) return rc;
     plan = w.plan;
   }
-  if ((rc = sas_resolve(p, t, plan, ws, ws_bytes, stream))) return rc;
+  const bool tiles = kv_grad && L.tile;
+  const bool use_inv = tiles && p->scenario == 3 && L.cmp_rows > 0;
+  uint32_t* inv = use_inv ? reinterpret_cast<uint32_t*>(base + L.off_inv) : nullptr;
+  if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, true, inv, L.cmp_rows))) return rc;
   const SasFwdArgs a = fwd_args(p, target);
-  const bool f16 = p->q_dtype == SAS_DT_FP16;
-  if (f16)
-    hipLaunchKernelGGL(sas::bwd_prep_kernel<1>, dim3(T * ((H + 3) / 4)), dim3(256), 0, s, a, p->head_dim_qk, plan,
-                       static_cast<const int2*>(w.tok),
-                       static_cast<const uint16_t*>(dout), static_cast<const uint16_t*>(t->out),
-                       t->lse, dlse, t->sinks, dterm, sterm, dq);
-  else
-    hipLaunchKernelGGL(sas::bwd_prep_kernel<0>, dim3(T * ((H + 3) / 4)), dim3(256), 0, s, a, p->head_dim_qk, plan,
-                       static_cast<const int2*>(w.tok),
-                       static_cast<const uint16_t*>(dout), static_cast<const uint16_t*>(t->out),
-                       t->lse, dlse, t->sinks, dterm, sterm, dq);
+  const bool f16 = p->q_dtype == SAS_DT_FP16, d576 = p->head_dim_qk == 576;
+  const uint16_t* q = static_cast<const uint16_t*>(t->q);
+  const uint16_t* go = static_cast<const uint16_t*>(dout);
+  const int2* tok = w.tok;
+  const uint64_t* addr = w.addr;
+  int* flags = tiles ? reinterpret_cast<int*>(base + L.off_flags) : nullptr;
+  hipLaunchKernelGGL(f16 ? &sas::bwd_prep_kernel<1> : &sas::bwd_prep_kernel<0>,
+                     dim3(T * ((H + 3) / 4)), dim3(256), 0, s, a, p->head_dim_qk, plan, tok, go,
+                     static_cast<const uint16_t*>(t->out), t->lse, dlse, t->sinks, dterm, sterm, dq,
+                     flags);
   if ((rc = launch_status())) return rc;
   const dim3 grid(a.unit_cap * ((H + sas::BW_HEADS - 1) / sas::BW_HEADS));
   typedef void (*bwd_fn_t)(SasFwdArgs, const uint16_t*, const uint16_t*, const uint64_t*,
-                           const int2*, const float*, const float*, const int*, float*);
-  bwd_fn_t fn = p->head_dim_qk == 576 ? (f16 ? &sas::bwd_dq_kernel<576, 1> : &sas::bwd_dq_kernel<576, 0>)
-                                      : (f16 ? &sas::bwd_dq_kernel<512, 1> : &sas::bwd_dq_kernel<512, 0>);
-  hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, a, static_cast<const uint16_t*>(t->q),
-                     static_cast<const uint16_t*>(dout), static_cast<const uint64_t*>(w.addr),
-                     static_cast<const int2*>(w.tok), static_cast<const float*>(t->lse),
-                     static_cast<const float*>(dterm), plan, dq);
-  if ((rc = launch_status())) return rc;
-  if (d_ori_kv || d_cmp_kv) {  // the KV pools' gradient (accumulated into the buffers)
-    const dim3 gkv(a.unit_cap);  // one workgroup per work unit, all heads
+                           const int2*, const float*, const float*, const int*, float*,
+                           sas::SasBwdSpill);
+  const bwd_fn_t fn = tiles ? (d576 ? (f16 ? &sas::bwd_dq_kernel<576, 1, true> : &sas::bwd_dq_kernel<576, 0, true>)
+                                    : (f16 ? &sas::bwd_dq_kernel<512, 1, true> : &sas::bwd_dq_kernel<512, 0, true>))
+                            : (d576 ? (f16 ? &sas::bwd_dq_kernel<576, 1, false> : &sas::bwd_dq_kernel<576, 0, false>)
+                                    : (f16 ? &sas::bwd_dq_kernel<512, 1, false> : &sas::bwd_dq_kernel<512, 0, false>));
+  sas::SasBwdSpill sp = {};
+  sas::SasTileArgs ta = {};
+  if (tiles) {
+    sp.stride = L.stride;
+    sp.row_bytes = L.row_bytes;
+    sp.data = reinterpret_cast<uint8_t*>(base + L.off_spill);
+    sp.flags = flags;
+    ta.q_prefix = t->q_prefix;
+    ta.act_q = t->act_q_lens;
+    ta.seqused_kv = t->seqused_kv;
+    ta.ori_bt = t->ori_block_table;
+    ta.cmp_bt = t->cmp_block_table;
+    ta.inv = inv;
+    ta.cmp_rows = L.cmp_rows;
+    // one workgroup per CU (its LDS), a multiple of the XCDs
+    ta.workers = std::max(8, query_num_cus() / 8 * 8);
+    ta.item_cap = (int)L.item_cap;
+    ta.want_ori = d_ori_kv != nullptr;
+    ta.want_cmp = L.cmp_rows > 0 && d_cmp_kv != nullptr;
+    ta.items = reinterpret_cast<int4*>(base + L.off_items);
+  }
+  // the tokens in runs that the spill holds (one run where nothing is spilled)
+  for (int t0 = 0; t0 < T; t0 += L.chunk_tokens) {
+    sp.t0 = t0;
+    sp.t1 = std::min(T, t0 + L.chunk_tokens);
+    hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, a, q, go, addr, tok,
+                       static_cast<const float*>(t->lse), static_cast<const float*>(dterm), plan, dq, sp);
+    if ((rc = launch_status())) return rc;
+    if (!tiles) break;
+    hipLaunchKernelGGL(sas::bwd_items_kernel, dim3(1), dim3(1024), 0, s, a, ta, sp, plan);
+    if ((rc = launch_status())) return rc;
+    typedef void (*tile_fn_t)(SasFwdArgs, sas::SasTileArgs, sas::SasBwdSpill, const uint16_t*,
+                              const uint16_t*, const int2*, const int*, float*, float*);
+    const tile_fn_t tf = d576 ? (f16 ? &sas::bwd_dkv_tile_kernel<576, 1> : &sas::bwd_dkv_tile_kernel<576, 0>)
+                              : (f16 ? &sas::bwd_dkv_tile_kernel<512, 1> : &sas::bwd_dkv_tile_kernel<512, 0>);
+    hipLaunchKernelGGL(tf, dim3(ta.workers), dim3(sas::TK_NT), 0, s, a, ta, sp,
+                       q, go, tok, plan, d_ori_kv, d_cmp_kv);
+    if ((rc = launch_status())) return rc;
+  }
+  if (kv_grad) {  // the KV pools' gradient (accumulated into the buffers)
+    // what the tiles leave: everything without them; the compressed rows where they are
+    // not covered; the tokens marked for an infinity or a NaN
+    const int mode = !tiles ? 0 : p->scenario >= 2 && L.cmp_rows == 0 ? 1 : 2;
+    const dim3 gkv(mode == 2 ? std::min(a.unit_cap, std::max(1, query_num_cus())) : a.unit_cap);
     typedef void (*dkv_fn_t)(SasFwdArgs, const uint16_t*, const uint16_t*, const uint64_t*,
                              const int*, const int2*, const float*, const float*, const int*,
-                             float*, float*);
-    dkv_fn_t kf = p->head_dim_qk == 576
-                      ? (f16 ? &sas::bwd_dkv_kernel<576, 1> : &sas::bwd_dkv_kernel<576, 0>)
-                      : (f16 ? &sas::bwd_dkv_kernel<512, 1> : &sas::bwd_dkv_kernel<512, 0>);
-    hipLaunchKernelGGL(kf, gkv, dim3(256), 0, s, a, static_cast<const uint16_t*>(t->q),
-                       static_cast<const uint16_t*>(dout), static_cast<const uint64_t*>(w.addr),
-                       static_cast<const int*>(w.rows), static_cast<const int2*>(w.tok),
+                             float*, float*, int, const int*);
+    const dkv_fn_t kf = d576 ? (f16 ? &sas::bwd_dkv_kernel<576, 1> : &sas::bwd_dkv_kernel<576, 0>)
+                             : (f16 ? &sas::bwd_dkv_kernel<512, 1> : &sas::bwd_dkv_kernel<512, 0>);
+    hipLaunchKernelGGL(kf, gkv, dim3(256), 0, s, a, q, go, addr, static_cast<const int*>(w.rows), tok,
                        static_cast<const float*>(t->lse), static_cast<const float*>(dterm), plan,
-                       d_ori_kv, p->scenario >= 2 ? d_cmp_kv : nullptr);
+                       d_ori_kv, p->scenario >= 2 ? d_cmp_kv : nullptr, mode,
+                       static_cast<const int*>(flags));
     if ((rc = launch_status())) return rc;
   }
   hipLaunchKernelGGL(sas::bwd_dsink_kernel, dim3(H), dim3(256), 0, s, T, H,

@@ -132,6 +132,83 @@ SAS_HD static inline SasWsLayout sas_ws_layout(int64_t T, int64_t K, int64_t H, 
   return W;
 }
 
+// ---- backward workspace: the forward's, then (bytes, each region 256-B aligned) ----
+// The KV pools' gradient by key tiles (bwd_dkv_tile_kernel) reads every row's P and dS
+// back from memory: the dq kernel spills them, one record per list position (2 B dS and
+// 2 B P per head, heads padded to whole 32-head chunks).  The spill is bounded: the
+// tokens are taken in runs of chunk_tokens.
+#define SAS_BWD_KEYS 128                          // keys per tile item
+#define SAS_BWD_SPILL_BYTES ((size_t)2 << 30)     // spill bound (at least one token)
+#define SAS_BWD_MIN_GROUP 8                       // fewest tokens per tile item
+#define SAS_BWD_MAX_B 2048                        // sequences the item list handles
+// Tiles for compressed rows when the table holds at most this times K rows: a tile visit
+// (a token against 128 keys) costs about 17 ns of the chip's time, an atomic row 1.75 ns
+// (576 adds at 330 G/s), so the two meet where a token lists about 10 of 128 rows; at a
+// sixth of them (21) the tiles are ahead, with room for lists that are shorter than K.
+#define SAS_BWD_DENSE 6
+
+struct SasBwdLayout {
+  size_t off_dterm, off_sterm;  // D and the sink term per (token, head)
+  size_t base_total;            // without the KV pools' gradient
+  size_t off_flags, off_inv, off_items, off_spill, total;
+  int tile;           // key tiles for the window rows
+  int cmp_rows;       // compressed rows per sequence covered by tiles (0: none)
+  int stride;         // spilled list positions per token
+  int row_bytes;      // bytes per spilled position
+  int chunk_tokens;   // tokens per run
+  int64_t item_cap;
+};
+
+SAS_HD static inline SasBwdLayout sas_bwd_layout(size_t fwd_total, int64_t T, int64_t B, int64_t H,
+                                                 int scenario, int64_t win_left, int64_t K,
+                                                 int64_t cmp_cap) {
+  SasBwdLayout L;
+  const size_t th = (size_t)(T > 0 ? T : 1) * (size_t)H;
+  L.off_dterm = fwd_total;
+  L.off_sterm = L.off_dterm + sas_align256(th * 4);
+  L.base_total = L.off_sterm + sas_align256(th * 4);
+  L.row_bytes = (int)((H + 31) / 32) * 128;
+  // tiles pay where several tokens of a sequence share their rows
+  L.tile = T >= 8 * B && B <= SAS_BWD_MAX_B;
+  const int64_t full = sas_row_list_stride(win_left, K, scenario);
+  int64_t stride = sas_row_list_stride(win_left, 0, 1);
+  // Compressed rows: a tile visits every token that may list one of its 128 rows, so
+  // it pays while a token lists a fair share of them; list positions fit 16 bits.
+  L.cmp_rows = 0;
+  if (L.tile && scenario >= 2 && full < 65536 && (scenario == 2 || cmp_cap <= SAS_BWD_DENSE * K)) {
+    L.cmp_rows = (int)cmp_cap;
+    stride = full;
+  }
+  const size_t per_token = (size_t)stride * (size_t)L.row_bytes;
+  if (per_token > SAS_BWD_SPILL_BYTES) L.tile = L.cmp_rows = 0;
+  L.stride = (int)stride;
+  L.off_flags = L.off_inv = L.off_items = L.off_spill = L.total = L.base_total;
+  L.chunk_tokens = (int)(T > 0 ? T : 1);
+  L.item_cap = 0;
+  if (!L.tile) return L;
+  int64_t chunk = (int64_t)(SAS_BWD_SPILL_BYTES / per_token);
+  if (chunk < 1) chunk = 1;
+  const int64_t runs = (T + chunk - 1) / chunk;
+  chunk = ((T + runs - 1) / runs + 63) / 64 * 64;
+  if (chunk > T) chunk = T;
+  L.chunk_tokens = (int)chunk;
+  // groups of a run: at most chunk / group + one partial group per sequence; tiles of a
+  // group: those its window span and its compressed rows touch
+  const int64_t groups = chunk / SAS_BWD_MIN_GROUP + B + 1;
+  const int64_t tiles = (win_left + 64) / SAS_BWD_KEYS + 2 +
+                        (L.cmp_rows + SAS_BWD_KEYS - 1) / SAS_BWD_KEYS;
+  L.item_cap = groups * tiles;
+  L.off_flags = L.total;
+  L.total += sas_align256((size_t)(T + 1) * 4);
+  L.off_inv = L.total;
+  if (scenario == 3) L.total += sas_align256((size_t)T * (size_t)L.cmp_rows * 4);
+  L.off_items = L.total;
+  L.total += sas_align256((size_t)(L.item_cap + 1) * 16);
+  L.off_spill = L.total;
+  L.total += sas_align256(((size_t)chunk * (size_t)stride + 1) * (size_t)L.row_bytes);
+  return L;
+}
+
 // ---- kernel parameter blocks (passed by value) ----
 struct SasPlanArgs {
   int32_t T, B, scenario, win_left, cmp_ratio, K, H, target;

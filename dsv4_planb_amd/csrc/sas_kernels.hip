@@ -414,6 +414,11 @@ struct SasResolveArgs {
   const float* ori_scale;
   const float* cmp_scale;
   float* scale;           // fp8: s, then (T * list_stride on) 1 / s; nullptr for 16-bit KV
+  // INV: scenario 3's inverse list, [T][inv_rows]: for compressed row j of the token's
+  // sequence, the list position of its first occurrence (low 16 bits) and how often
+  // it is listed (high 16 bits; 0: not).  Entries below the token's threshold are set.
+  uint32_t* inv;
+  int inv_rows;
 };
 
 // List positions [lo, hi) of token t (its window rows, then its compressed rows)
@@ -434,6 +439,7 @@ struct SasResolveArgs {
 // reuses its metadata).  Where the call's q_prefix / act_q no longer give the token
 // to batch b at position s (or give a token the plan left unowned to its candidate
 // batch), the token is refused: nwin_live = -1, nothing is resolved.
+template <bool INV>
 __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, int t, int lo, int hi,
                             RsShared& sh, const SasResolveArgs& r, int& nwin_live) {
   const int tid = threadIdx.x;
@@ -533,6 +539,15 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
     return n;
   }
   const int limit = max(min(a.K, thr), 0);  // golden.py:48
+  typedef __attribute__((address_space(1))) uint32_t g_u32;
+  g_u32* inv = nullptr;
+  if constexpr (INV) {
+    if (r.inv) {
+      inv = (g_u32*)(uintptr_t)(r.inv + (size_t)t * r.inv_rows);
+      for (int i = tid; i < min(thr, r.inv_rows); i += RS_NT) inv[i] = 0;
+      __syncthreads();  // the zeros are in place before the first count below
+    }
+  }
   // Passes of RS_PER slabs of RS_NT slots; the terminator, the survivors and their
   // slot-order positions come from ballots and two LDS exchanges per pass.
   int emitted = 0;  // compressed rows found so far (block-uniform)
@@ -624,6 +639,11 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
         if (out) out[p] = code[k];
         if (sout) put_scale(p, sc[k]);
         aout[p] = code_addr(code[k], r.cmp_kv, a.cmp_block_size, a.cmp_block_stride, a.cmp_row_stride, r.esz);
+        if constexpr (INV) {
+          if (inv && v[k] < r.inv_rows &&
+              __hip_atomic_fetch_add(inv + v[k], 1u << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (1u << 16))
+            __hip_atomic_fetch_or(inv + v[k], (uint32_t)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
       }
     emitted = total;
     if (term < limit) break;  // the list ended in this pass
@@ -633,6 +653,7 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
 }
 
 // One workgroup (RS_NT threads) per token: its whole list.
+template <bool INV>
 __global__ __launch_bounds__(RS_NT) void resolve_kernel(SasFwdArgs a, const int* __restrict__ plan,
                                                         SasResolveArgs r) {
   __shared__ RsShared sh;
@@ -642,7 +663,7 @@ __global__ __launch_bounds__(RS_NT) void resolve_kernel(SasFwdArgs a, const int*
   const bool plan_ok = plan_matches(plan, a);
   const int* tk = plan + SAS_PLAN_HDR + (size_t)t * SAS_TOK_W;
   int nwin = 0;
-  const int n = resolve_rows(a, tk, plan_ok, t, 0, a.list_stride, sh, r, nwin);
+  const int n = resolve_rows<INV>(a, tk, plan_ok, t, 0, a.list_stride, sh, r, nwin);
   if (threadIdx.x == 0 && r.tok) r.tok[t] = make_int2(nwin, nwin < 0 ? 0 : n);
 }
 

@@ -201,8 +201,11 @@ int sas_attend_timed(const sas_params_t* p, const sas_tensors_t* t, const int32_
  * blocks) into which the pools' gradient is ADDED (dK over head_dim_qk, dV over the
  * first head_dim_v dimensions; rows read as zeros get nothing): zero them first.
  * Rows read by several tokens are summed with fp32 atomics (order not fixed).
- * d_cmp_kv is ignored in scenario 1.  workspace: sas_backward_workspace_size bytes. */
+ * d_cmp_kv is ignored in scenario 1.  workspace: sas_backward_workspace_size bytes,
+ * or, for calls that ask for no pool gradient (both NULL), the smaller
+ * sas_backward_workspace_size_for(p, 0, ...). */
 int sas_backward_workspace_size(const sas_params_t* p, size_t* bytes);
+int sas_backward_workspace_size_for(const sas_params_t* p, int kv_grad, size_t* bytes);
 int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan,
                  const void* dout, const float* dlse /* [T, H] or NULL */, float* dq,
                  float* dsinks, float* d_ori_kv /* or NULL */, float* d_cmp_kv /* or NULL */,
