@@ -16,6 +16,7 @@
 #include "sas_common.h"
 #include "sas_kernels.hip"
 #include "sas_attend.hip"
+#include "sas_attend_narrow.hip"
 #include "sas_backward.hip"
 #include "sas_backward_tile.hip"
 
@@ -166,19 +167,11 @@ attend_fn_t attend_ptr(bool f16, bool nt) {
   return nt ? attend_ptr<DQK, true, KV8>(f16) : attend_ptr<DQK, false, KV8>(f16);
 }
 
-// Decode-like calls (at most 4 query tokens per sequence on average) read each KV
-// row for one token only: their gather uses non-temporal loads.  Prefill-like calls,
-// where nearby tokens share most of their rows, keep the default cache policy.
-attend_fn_t pick_attend(const sas_params_t* p) {
-  const bool f16 = p->q_dtype == SAS_DT_FP16;
-  const bool nt = (int64_t)p->total_tokens <= 4 * (int64_t)p->batch;
-  const bool kv8 = p->kv_dtype == SAS_DT_FP8E4M3;
-  if (p->head_dim_qk == 576)
-    return kv8 ? attend_ptr<576, true>(f16, nt) : attend_ptr<576, false>(f16, nt);
-  return kv8 ? attend_ptr<512, true>(f16, nt) : attend_ptr<512, false>(f16, nt);
+template <int DQK>
+attend_fn_t narrow_ptr(bool f16, bool nt) {
+  return nt ? (f16 ? &sas::attend_narrow_kernel<DQK, 1, true> : &sas::attend_narrow_kernel<DQK, 0, true>)
+            : (f16 ? &sas::attend_narrow_kernel<DQK, 1, false> : &sas::attend_narrow_kernel<DQK, 0, false>);
 }
-
-int launch_status() { return hipGetLastError() == hipSuccess ? SAS_OK : SAS_ERR_LAUNCH; }
 
 // Does the forward let every unit resolve its own rows?  With at most as many
 // tokens as target units every unit starts in the first wave of workgroups, and
@@ -187,6 +180,31 @@ int launch_status() { return hipGetLastError() == hipSuccess ? SAS_OK : SAS_ERR_
 bool fused_resolution(const sas_params_t* p, int target) {
   return (int64_t)p->total_tokens <= (int64_t)target;
 }
+
+// At most 64 heads (16-bit KV) and more tokens than target units: the two-wave kernel, two
+// of whose workgroups share a CU, so that one's start and epilogue run under the other's
+// tiles.  Where every unit starts at once nothing runs beside it, and the four-wave
+// kernel's wider gather and resolution win (32 sequences of 4k to 32k tokens, 64 heads,
+// top-k 512, a graph replay: 32.6 us against 35.2 us with two waves; 101 tokens of 16
+// heads, top-k 1024, an eager step with its plan: 125 against 147 us).
+bool narrow_heads(const sas_params_t* p, int target) {
+  return p->num_heads_q <= 64 && p->kv_dtype != SAS_DT_FP8E4M3 && !fused_resolution(p, target);
+}
+
+// Decode-like calls (at most 4 query tokens per sequence on average) read each KV
+// row for one token only: their gather uses non-temporal loads.  Prefill-like calls,
+// where nearby tokens share most of their rows, keep the default cache policy.
+attend_fn_t pick_attend(const sas_params_t* p, int target) {
+  const bool f16 = p->q_dtype == SAS_DT_FP16;
+  const bool nt = (int64_t)p->total_tokens <= 4 * (int64_t)p->batch;
+  const bool kv8 = p->kv_dtype == SAS_DT_FP8E4M3;
+  if (narrow_heads(p, target)) return p->head_dim_qk == 576 ? narrow_ptr<576>(f16, nt) : narrow_ptr<512>(f16, nt);
+  if (p->head_dim_qk == 576)
+    return kv8 ? attend_ptr<576, true>(f16, nt) : attend_ptr<576, false>(f16, nt);
+  return kv8 ? attend_ptr<512, true>(f16, nt) : attend_ptr<512, false>(f16, nt);
+}
+
+int launch_status() { return hipGetLastError() == hipSuccess ? SAS_OK : SAS_ERR_LAUNCH; }
 
 // The attention kernel over the plan's units.  resolve: each unit first resolves
 // its own rows (the resolver stage is then not launched).  With events, the
@@ -204,7 +222,7 @@ int launch_attend(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
   // no workgroup past the last unit is launched only to exit; otherwise the grid is
   // the plan's unit capacity and those past the plan's count exit at once.
   const int grid = resolve ? target : a.unit_cap;
-  hipExtLaunchKernelGGL(pick_attend(p), dim3(grid), dim3(256), 0, (hipStream_t)stream,
+  hipExtLaunchKernelGGL(pick_attend(p, target), dim3(grid), dim3(narrow_heads(p, target) ? sas::NW_NT : 256), 0, (hipStream_t)stream,
                         (hipEvent_t)start_event, (hipEvent_t)stop_event, 0, a,
                         static_cast<const uint16_t*>(t->q), static_cast<const uint64_t*>(w.addr),
                         static_cast<const float*>(w.scale), static_cast<const int2*>(w.tok),

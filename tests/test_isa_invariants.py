@@ -99,3 +99,26 @@ def test_attention_tile_loop_keeps_dmas_in_flight(asm):
         assert not waits, (name[:60], waits[:3])
         checked += 1
     assert checked == 8  # {bf16, fp16} x {streaming, cached gather} x {16-bit, fp8 KV}
+
+
+def test_narrow_tile_loop_keeps_dmas_in_flight(asm):
+    """The two-wave attention kernel's loop: no full vector-memory wait either (a load
+    copied where two ways through the loop join, or a global LDS-direct load the compiler
+    counts, makes one)."""
+    checked = 0
+    for name, body in _kernels(asm):
+        if "attend_narrow_kernelILi576" not in name:
+            continue
+        labels = {m.group(1): i for i, l in enumerate(body) if (m := re.match(r"^(\.LBB\S+):", l))}
+        loops = []
+        for i, l in enumerate(body):
+            m = re.match(r"\s+s_c?branch\w*\s+(\.LBB\S+)", l)
+            if m and m.group(1) in labels and labels[m.group(1)] < i:
+                a = labels[m.group(1)]
+                loops.append((sum("v_mfma" in body[j] for j in range(a, i)), a, i))
+        n_mfma, a, b = max(loops)
+        assert n_mfma >= 50, (name[:60], n_mfma)
+        waits = [body[j].strip() for j in range(a, b) if re.search(r"s_waitcnt vmcnt\(0\)", body[j])]
+        assert not waits, (name[:60], waits[:3])
+        checked += 1
+    assert checked == 4
