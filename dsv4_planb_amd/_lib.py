@@ -30,7 +30,8 @@ SYMBOLS = (
     "sas_debug_rows", "sas_graph_capture", "sas_graph_launch", "sas_graph_destroy",
     "sas_metadata_legacy", "sas_forward_noalloc", "sas_attend_timed",
     "sas_backward_workspace_size",
-    "sas_backward_workspace_size_for", "sas_backward", "sas_debug_lists",
+    "sas_backward_workspace_size_for", "sas_backward", "sas_debug_lists", "sas_forward_cu",
+    "sas_call_sizes",
 )
 SAS_SCRATCH_BYTES = 160 << 20  # include/sas.h: the fixed workspace of sas_forward_noalloc
 
@@ -101,10 +102,11 @@ def load():
         lib.sas_version.argtypes, lib.sas_version.restype = [], I
         lib.sas_validate.argtypes, lib.sas_validate.restype = [PP], I
         lib.sas_workspace_size.argtypes = [PP, ctypes.POINTER(S)]
+        lib.sas_call_sizes.argtypes = [PP, P]
         lib.sas_plan_size.argtypes = [PP, ctypes.POINTER(S)]
         lib.sas_target_units.argtypes = [PP, ctypes.POINTER(ctypes.c_int32)]
         lib.sas_plan.argtypes = [PP, P, P, P, P, S, P]
-        for fn in ("sas_forward", "sas_resolve", "sas_attend", "sas_combine"):
+        for fn in ("sas_forward", "sas_forward_cu", "sas_resolve", "sas_attend", "sas_combine"):
             getattr(lib, fn).argtypes = [PP, PT, P, P, S, P]
         lib.sas_debug_rows.argtypes = [PP, P, P, P, P]
         lib.sas_debug_lists.argtypes = [PP, P, P, P, P, P]

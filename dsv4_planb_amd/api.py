@@ -70,7 +70,16 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _dev_i32(t: torch.Tensor, device) -> torch.Tensor:
+    # (the usual case first: a tensor that needs nothing costs no dispatch)
+    if t.dtype is torch.int32 and t.device == device and t.is_contiguous():
+        return t
     return t.to(device=device, dtype=torch.int32).contiguous()
+
+
+def _dev_f32(t: torch.Tensor, device) -> torch.Tensor:
+    if t.dtype is torch.float32 and t.device == device and t.is_contiguous():
+        return t
+    return t.to(device=device, dtype=torch.float32).contiguous()
 
 
 def _paged_strides(kv: torch.Tensor, D: int, name: str):
@@ -78,26 +87,28 @@ def _paged_strides(kv: torch.Tensor, D: int, name: str):
         raise ValueError(f"{name} must be paged [block_num, block_size, N2, D], got {tuple(kv.shape)}")
     if kv.shape[3] != D:
         raise ValueError(f"{name} head dim {kv.shape[3]} != q head dim {D}")
-    if kv.stride(3) != 1:
+    stride = kv.stride()
+    if stride[3] != 1:
         raise ValueError(f"{name} rows must be contiguous in the head dim")
-    return int(kv.stride(0)), int(kv.stride(1))
+    return stride[0], stride[1]
 
 
 def _stream_handle(device) -> ctypes.c_void_p:
+    if device.index is not None:  # (without building a Stream object)
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(device.index))
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
-def _check_plan_record(metadata: torch.Tensor, p: SasParams, host_lens) -> None:
+def _check_plan_record(metadata: torch.Tensor, p: SasParams, host_lens, target: int) -> None:
     """Raise ``ValueError`` when the plan's own record (written by the metadata op,
     valid while the tensor is unmodified) names other arguments than this call:
     the host-side counterpart of the kernels' check, with the reason spelled out.
-    host_lens: the call's (q_prefix, act_q) on the host, or None when they are on
-    the device only (then the device check covers them, without a host sync)."""
+    host_lens: the call's (q_prefix, act_q) on the host (or a function that returns
+    them), or None when they are on the device only (then the device check covers
+    them, without a host sync); target: the call's balance target."""
     rec = getattr(metadata, "_sas_plan", None)
     if rec is None or rec.get("version") != metadata._version:
         return
-    target = ctypes.c_int32()
-    _lib.check(_lib.load().sas_target_units(ctypes.byref(p), ctypes.byref(target)), "sas_target_units")
     diffs = []
 
     def cmp(name, planned, called):
@@ -112,9 +123,10 @@ def _check_plan_record(metadata: torch.Tensor, p: SasParams, host_lens) -> None:
         cmp("cmp_ratio", rec["cmp_ratio"], int(p.cmp_ratio))
     if p.scenario == 3:
         cmp("topk", rec["K"], int(p.topk))
-    cmp("work units (core_num)", rec["target"], int(target.value))
+    cmp("work units (core_num)", rec["target"], target)
     if not diffs and host_lens is not None and rec.get("q_prefix") is not None:
-        qp, aq = (x.to("cpu", torch.int64).reshape(-1) for x in host_lens)
+        lens = host_lens() if callable(host_lens) else host_lens
+        qp, aq = (x.to("cpu", torch.int64).reshape(-1) for x in lens)
         if not (torch.equal(qp, rec["q_prefix"]) and torch.equal(aq, rec["act_q"])):
             diffs.append("query layout (cu_seqlens_q / seqused_q) differs from the plan's")
     if diffs:
@@ -246,7 +258,8 @@ class SasLaunch:
         fn = getattr(lib, f"sas_{stage}")
         rc = fn(ctypes.byref(self.params), ctypes.byref(self.tensors), _ptr(self.plan),
                 _ptr(self.ws), self.ws.numel(), _stream_handle(self.device))
-        _lib.check(rc, f"sas_{stage}")
+        if rc:
+            _lib.check(rc, f"sas_{stage}")
 
 
 def build_launch(
@@ -276,9 +289,9 @@ def build_launch(
     host_lens=None,
 ) -> Tuple[SasLaunch, torch.Tensor, torch.Tensor]:
     """Validate, convert and lay out one call; returns (launch, out, lse).
-    host_lens: the call's (q_prefix, act_q) on the host where the caller has them,
-    for the check of a recorded plan (q_prefix / act_q_lens given as CPU tensors
-    serve as well)."""
+    host_lens: the call's (q_prefix, act_q) on the host where the caller has them (or
+    a function that returns them), for the check of a recorded plan (q_prefix /
+    act_q_lens given as CPU tensors serve as well)."""
     lib = _lib.load()
     dev = q_flat.device
     if dev.type != "cuda":
@@ -287,66 +300,54 @@ def build_launch(
     q_code = _torch_to_sas_dtype(q_flat.dtype)
     kv_code = _kv_dtype_code(ori_kv, q_code)
     q_flat = q_flat.contiguous()
-    ori_kv = ori_kv.to(dev)
+    if ori_kv.device != dev:
+        ori_kv = ori_kv.to(dev)
     obs, ors = _paged_strides(ori_kv, D, "ori_kv")
-    p = SasParams()
-    p.batch = int(q_prefix.numel())
-    p.total_tokens = T
-    p.num_heads_q = N1
-    p.num_heads_kv = int(ori_kv.shape[2])
-    p.head_dim_qk = D
-    p.head_dim_v = 512
-    p.ori_block_num, p.ori_block_size = int(ori_kv.shape[0]), int(ori_kv.shape[1])
     ori_bt = _dev_i32(ori_block_table, dev)
-    p.ori_table_len = int(ori_bt.shape[1])
-    p.ori_block_stride, p.ori_row_stride = obs, ors
     keep = [q_flat, ori_kv, ori_bt]
     cmp_bt = idx = None
+    cmp_block_num = cmp_block_size = cmp_table_len = 1
+    cbs = crs = D
     if scenario >= 2:
-        cmp_kv = cmp_kv.to(dev)
+        if cmp_kv.device != dev:
+            cmp_kv = cmp_kv.to(dev)
         if _kv_dtype_code(cmp_kv, q_code) != kv_code:
             raise ValueError("ori_kv and cmp_kv must share a dtype")
         cbs, crs = _paged_strides(cmp_kv, D, "cmp_kv")
         cmp_bt = _dev_i32(cmp_block_table, dev)
-        p.cmp_block_num, p.cmp_block_size = int(cmp_kv.shape[0]), int(cmp_kv.shape[1])
-        p.cmp_table_len = int(cmp_bt.shape[1])
-        p.cmp_block_stride, p.cmp_row_stride = cbs, crs
+        cmp_block_num, cmp_block_size = cmp_kv.shape[0], cmp_kv.shape[1]
+        cmp_table_len = cmp_bt.shape[1]
         keep += [cmp_kv, cmp_bt]
     else:
         cmp_kv = None
-        p.cmp_block_num = p.cmp_block_size = p.cmp_table_len = 1
-        p.cmp_block_stride = p.cmp_row_stride = D
     if scenario == 3:
         idx = _dev_i32(cmp_indices, dev).reshape(T, -1)
         keep.append(idx)
     # scenario 3: index slots per token; scenario 2: capacity of the per-token list
     # of causally valid compressed rows -- the rows the block table covers
-    p.topk = topk if scenario == 3 else (p.cmp_table_len * p.cmp_block_size if scenario == 2 else 0)
-    p.cmp_ratio = cmp_ratio
-    p.scenario = scenario
-    p.ori_win_left = ori_win_left
-    p.ori_win_right = 0
-    p.ori_mask_mode = 4
-    p.cmp_mask_mode = 3
-    p.q_dtype = q_code
-    p.kv_dtype = kv_code
-    p.softmax_scale = float(softmax_scale)
-    p.num_cus = int(core_num)
-    p.units_per_cu = int(units_per_cu)
-    rc = lib.sas_validate(ctypes.byref(p))
-    if rc == -6:  # heads: the reference raises ValueError for unsupported N1/N2 (api.py:279-282)
-        raise ValueError(f"num_heads_kv must be 1 and num_heads_q in [1, 128] "
-                         f"(got N1={N1}, N2={p.num_heads_kv}, D={D})")
-    if rc == -2 and D not in (512, 576):
-        raise ValueError(f"head_dim must be 512 or 576 (got {D})")
-    _lib.check(rc, "sparse_attn_sharedkv")
+    slots = topk if scenario == 3 else (cmp_table_len * cmp_block_size if scenario == 2 else 0)
+    # (the fields in the structure's order: one call instead of one per field)
+    p = SasParams(q_prefix.numel(), T, N1, ori_kv.shape[2], D, 512,
+                  ori_kv.shape[0], ori_kv.shape[1], ori_bt.shape[1],
+                  cmp_block_num, cmp_block_size, cmp_table_len, obs, ors, cbs, crs,
+                  slots, cmp_ratio, scenario, ori_win_left, 0, 4, 3, q_code, kv_code,
+                  float(softmax_scale), int(core_num), int(units_per_cu))
+    sizes = (ctypes.c_int64 * 3)()  # balance target, plan entries, workspace bytes
+    rc = lib.sas_call_sizes(ctypes.byref(p), sizes)
+    if rc:
+        if rc == -6:  # heads: the reference raises ValueError for unsupported N1/N2 (api.py:279-282)
+            raise ValueError(f"num_heads_kv must be 1 and num_heads_q in [1, 128] "
+                             f"(got N1={N1}, N2={p.num_heads_kv}, D={D})")
+        if rc == -2 and D not in (512, 576):
+            raise ValueError(f"head_dim must be 512 or 576 (got {D})")
+        _lib.check(rc, "sparse_attn_sharedkv")
 
     if host_lens is None and q_prefix.device.type == "cpu" and act_q_lens.device.type == "cpu":
         host_lens = (q_prefix, act_q_lens)
     qp = _dev_i32(q_prefix, dev)
     aq = _dev_i32(act_q_lens, dev)
     skv = _dev_i32(seqused_kv, dev)
-    snk = sinks.to(device=dev, dtype=torch.float32).contiguous()
+    snk = _dev_f32(sinks, dev)
     if snk.numel() != N1:
         raise ValueError(f"sinks must have {N1} entries (got {snk.numel()})")
     keep += [qp, aq, skv, snk]
@@ -354,10 +355,10 @@ def build_launch(
     if kv_code == _lib.DT_FP8E4M3:
         if ori_kv_scale is None or (scenario >= 2 and cmp_kv_scale is None):
             raise ValueError("float8 KV needs ori_kv_scale (and cmp_kv_scale)")
-        osc = ori_kv_scale.to(device=dev, dtype=torch.float32).contiguous()
+        osc = _dev_f32(ori_kv_scale, dev)
         keep.append(osc)
         if scenario >= 2:
-            csc = cmp_kv_scale.to(device=dev, dtype=torch.float32).contiguous()
+            csc = _dev_f32(cmp_kv_scale, dev)
             keep.append(csc)
     if out is None:
         out = torch.empty((T, N1, 512), dtype=q_flat.dtype, device=dev)
@@ -369,29 +370,21 @@ def build_launch(
     if metadata is not None:
         n = metadata.numel()
         if n != SAS_META_SIZE:  # anything but the reference table must be our plan
-            need = ctypes.c_size_t()
-            _lib.check(lib.sas_plan_size(ctypes.byref(p), ctypes.byref(need)), "sas_plan_size")
-            assert n == need.value, (
+            assert n == sizes[1], (
                 f"metadata must have {SAS_META_SIZE} int32 entries (reference table) or "
-                f"{need.value} (split-KV plan for these shapes); got {n}")
-            _check_plan_record(metadata, p, host_lens)
-            plan = metadata.to(device=dev, dtype=torch.int32).contiguous()
+                f"{sizes[1]} (split-KV plan for these shapes); got {n}")
+            _check_plan_record(metadata, p, host_lens, sizes[0])
+            plan = _dev_i32(metadata, dev)
             keep.append(plan)
-    ws_bytes = ctypes.c_size_t()
-    _lib.check(lib.sas_workspace_size(ctypes.byref(p), ctypes.byref(ws_bytes)), "sas_workspace_size")
-    ws = torch.empty(int(ws_bytes.value), dtype=torch.uint8, device=dev)
+    ws = torch.empty(sizes[2], dtype=torch.uint8, device=dev)
     keep.append(ws)
 
-    t = SasTensors()
-    t.q, t.ori_kv, t.ori_block_table = q_flat.data_ptr(), ori_kv.data_ptr(), ori_bt.data_ptr()
-    t.cmp_kv = cmp_kv.data_ptr() if cmp_kv is not None else None
-    t.cmp_block_table = cmp_bt.data_ptr() if cmp_bt is not None else None
-    t.cmp_sparse_indices = idx.data_ptr() if idx is not None else None
-    t.q_prefix, t.act_q_lens, t.seqused_kv = qp.data_ptr(), aq.data_ptr(), skv.data_ptr()
-    t.sinks = snk.data_ptr()
-    t.ori_kv_scale = osc.data_ptr() if osc is not None else None
-    t.cmp_kv_scale = csc.data_ptr() if csc is not None else None
-    t.out, t.lse = out.data_ptr(), lse.data_ptr()
+    t = SasTensors(
+        q_flat.data_ptr(), ori_kv.data_ptr(), ori_bt.data_ptr(),
+        None if cmp_kv is None else cmp_kv.data_ptr(), None if cmp_bt is None else cmp_bt.data_ptr(),
+        None if idx is None else idx.data_ptr(), qp.data_ptr(), aq.data_ptr(), skv.data_ptr(),
+        snk.data_ptr(), None if osc is None else osc.data_ptr(),
+        None if csc is None else csc.data_ptr(), out.data_ptr(), lse.data_ptr())
     launch = SasLaunch(p, t, keep, plan, ws, dev)
     launch.ori_kv, launch.cmp_kv = ori_kv, cmp_kv
     return launch, out, lse
@@ -562,6 +555,11 @@ def sparse_attn_sharedkv(
     if cu_seqlens_q is not None and cu_seqlens_q.device.type == "cpu":
         cu_host = cu_seqlens_q.to(torch.int64).reshape(-1)
     host_lens = None
+    grad = torch.is_grad_enabled() and any(
+        x is not None and x.requires_grad for x in (q, sinks, ori_kv, cmp_kv))
+    # without a gradient the forward takes the sequences' cumulative ends as they are
+    # (sas_forward_cu): no kernel to form their lengths
+    ends = False
     if layout_q == "TND":
         assert cu_seqlens_q is not None, "cu_seqlens_q is required for TND"
         cu = _dev_i32(cu_seqlens_q, dev)
@@ -569,7 +567,8 @@ def sparse_attn_sharedkv(
         T = q.shape[0]
         q_flat = q
         q_prefix = cu[:-1]
-        act_q = cu[1:] - cu[:-1]
+        ends = not grad
+        act_q = cu[1:] if ends else cu[1:] - cu[:-1]
         idx = cmp_sparse_indices if scenario == 3 else None
         if cu_host is not None:
             host_lens = (cu_host[:-1], cu_host[1:] - cu_host[:-1])
@@ -577,13 +576,21 @@ def sparse_attn_sharedkv(
         B, S, N1, D = q.shape
         T = B * S
         q_flat = q.reshape(T, N1, D)
-        q_prefix = torch.arange(B, dtype=torch.int32, device=dev) * S
-        act_q = torch.full((B,), S, dtype=torch.int32, device=dev)
-        host_lens = (torch.arange(B, dtype=torch.int64) * S, torch.full((B,), S, dtype=torch.int64))
         if cu_seqlens_q is not None:
+            q_prefix = torch.arange(B, dtype=torch.int32, device=dev) * S
             cu = _dev_i32(cu_seqlens_q, dev)
             act_q = cu[1:] - cu[:-1]
-            host_lens = (host_lens[0], cu_host[1:] - cu_host[:-1]) if cu_host is not None else None
+            if cu_host is not None:
+                host_lens = (torch.arange(B, dtype=torch.int64) * S, cu_host[1:] - cu_host[:-1])
+        else:
+            if grad:
+                q_prefix = torch.arange(B, dtype=torch.int32, device=dev) * S
+                act_q = torch.full((B,), S, dtype=torch.int32, device=dev)
+            else:
+                cu = torch.arange(B + 1, dtype=torch.int32, device=dev) * S
+                q_prefix, act_q, ends = cu[:-1], cu[1:], True
+            host_lens = lambda: (torch.arange(B, dtype=torch.int64) * S,  # noqa: E731
+                                 torch.full((B,), S, dtype=torch.int64))
         idx = None
         if scenario == 3:
             ci = cmp_sparse_indices
@@ -604,8 +611,6 @@ def sparse_attn_sharedkv(
         metadata=metadata, scenario=scenario, topk=K, cmp_ratio=cmp_ratio_eff,
         ori_win_left=ori_win_left, softmax_scale=softmax_scale, core_num=core_num,
         ori_kv_scale=ori_kv_scale, cmp_kv_scale=cmp_kv_scale, host_lens=host_lens)
-    grad = torch.is_grad_enabled() and any(
-        x is not None and x.requires_grad for x in (q, sinks, ori_kv, cmp_kv))
     if grad:
         if ori_kv.dtype == torch.float8_e4m3fn:
             raise NotImplementedError("the backward supports 16-bit KV pools only")
@@ -613,7 +618,7 @@ def sparse_attn_sharedkv(
     else:
         launch, out, lse = build_launch(q_flat=q_flat, sinks=sinks, ori_kv=ori_kv, cmp_kv=cmp_kv,
                                         **spec)
-        launch.run()
+        launch.run("forward_cu" if ends else "forward")
 
     if layout_q == "BSND":
         out = out.reshape(B, S, out.shape[1], out.shape[2])

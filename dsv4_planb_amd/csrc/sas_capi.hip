@@ -72,7 +72,7 @@ SasFwdArgs fwd_args(const sas_params_t* p, int target) {
   return a;
 }
 
-SasPlanArgs plan_args(const sas_params_t* p, int target) {
+SasPlanArgs plan_args(const sas_params_t* p, int target, bool cu_ends = false) {
   SasPlanArgs a;
   a.T = p->total_tokens;
   a.B = p->batch;
@@ -82,6 +82,7 @@ SasPlanArgs plan_args(const sas_params_t* p, int target) {
   a.K = list_k(p);
   a.H = p->num_heads_q;
   a.target = target;
+  a.cu_ends = cu_ends;
   return a;
 }
 
@@ -135,10 +136,12 @@ typedef void (*attend_fn_t)(SasFwdArgs, const uint16_t*, const uint64_t*, const 
                             sas::SasResolveArgs);
 
 // Resolution's inputs and outputs in the workspace.
-sas::SasResolveArgs resolve_args(const sas_params_t* p, const sas_tensors_t* t, const Ws& w) {
+sas::SasResolveArgs resolve_args(const sas_params_t* p, const sas_tensors_t* t, const Ws& w,
+                                 bool cu_ends = false) {
   sas::SasResolveArgs r;
   r.q_prefix = t->q_prefix;
   r.act_q = t->act_q_lens;
+  r.cu_ends = cu_ends;
   r.seqused_kv = t->seqused_kv;
   r.ori_bt = t->ori_block_table;
   r.idx = t->cmp_sparse_indices;
@@ -211,10 +214,10 @@ int launch_status() { return hipGetLastError() == hipSuccess ? SAS_OK : SAS_ERR_
 // dispatch itself records its start and end into them.
 int launch_attend(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, const Ws& w,
                   int target, sas_stream_t stream, void* start_event, void* stop_event,
-                  bool resolve, uint64_t* stamps = nullptr) {
+                  bool resolve, uint64_t* stamps = nullptr, bool cu_ends = false) {
   SasFwdArgs a = fwd_args(p, target);
   a.stamps = stamps;
-  sas::SasResolveArgs r = resolve_args(p, t, w);
+  sas::SasResolveArgs r = resolve_args(p, t, w, cu_ends);
   if (!resolve) r.addr = nullptr;
   r.rows = nullptr;  // the forward needs addresses only (sas_resolve also writes the codes)
   // With at most `target` tokens (the units resolve their own rows) the planner makes
@@ -235,7 +238,7 @@ int launch_attend(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
 // only; the backward and sas_debug_rows read the codes).  inv: also the inverse lists.
 int resolve_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
                   size_t ws_bytes, sas_stream_t stream, bool codes, uint32_t* inv = nullptr,
-                  int inv_rows = 0) {
+                  int inv_rows = 0, bool cu_ends = false) {
   int rc = sas_validate(p);
   if (rc) return rc;
   if ((rc = check_tensors(p, t))) return rc;
@@ -244,7 +247,7 @@ int resolve_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
   if ((rc = carve(p, ws, ws_bytes, target, &w))) return rc;
   if (!plan) plan = w.plan;
   if (p->total_tokens == 0) return SAS_OK;
-  sas::SasResolveArgs r = resolve_args(p, t, w);
+  sas::SasResolveArgs r = resolve_args(p, t, w, cu_ends);
   if (!codes) r.rows = nullptr;
   r.inv = inv;
   r.inv_rows = inv_rows;
@@ -282,7 +285,7 @@ int combine_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
 }
 
 int forward_impl(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
-                 size_t ws_bytes, sas_stream_t stream, int32_t* status_out) {
+                 size_t ws_bytes, sas_stream_t stream, int32_t* status_out, bool cu_ends = false) {
   int rc = sas_validate(p);
   if (rc) return rc;
   if ((rc = check_tensors(p, t))) return rc;
@@ -292,15 +295,15 @@ int forward_impl(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
   if (p->total_tokens == 0) return SAS_OK;
   if (!plan) {
     hipLaunchKernelGGL(sas::plan_kernel, dim3(1), dim3(sas::PLAN_NT), 0, (hipStream_t)stream,
-                       plan_args(p, target), t->q_prefix, t->act_q_lens, t->seqused_kv, w.plan);
+                       plan_args(p, target, cu_ends), t->q_prefix, t->act_q_lens, t->seqused_kv, w.plan);
     if ((rc = launch_status())) return rc;
     plan = w.plan;
   }
   if (fused_resolution(p, target)) {
-    if ((rc = launch_attend(p, t, plan, w, target, stream, nullptr, nullptr, true))) return rc;
+    if ((rc = launch_attend(p, t, plan, w, target, stream, nullptr, nullptr, true, nullptr, cu_ends))) return rc;
   } else {
-    if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, false))) return rc;
-    if ((rc = launch_attend(p, t, plan, w, target, stream, nullptr, nullptr, false))) return rc;
+    if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, false, nullptr, 0, cu_ends))) return rc;
+    if ((rc = launch_attend(p, t, plan, w, target, stream, nullptr, nullptr, false, nullptr, cu_ends))) return rc;
   }
   return combine_stage(p, t, plan, ws, ws_bytes, stream, status_out);
 }
@@ -455,6 +458,23 @@ int sas_combine(const sas_params_t* p, const sas_tensors_t* t, const int32_t* pl
 int sas_forward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
                 size_t ws_bytes, sas_stream_t stream) {
   return forward_impl(p, t, plan, ws, ws_bytes, stream, nullptr);
+}
+
+int sas_forward_cu(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
+                   size_t ws_bytes, sas_stream_t stream) {
+  return forward_impl(p, t, plan, ws, ws_bytes, stream, nullptr, true);
+}
+
+int sas_call_sizes(const sas_params_t* p, int64_t* sizes) {
+  const int rc = sas_validate(p);
+  if (rc) return rc;
+  if (!sizes) return SAS_ERR_NULL;
+  const int target = target_units(p);
+  sizes[0] = target;
+  sizes[1] = sas_plan_layout(p->total_tokens, target).total;
+  sizes[2] = (int64_t)sas_ws_layout(p->total_tokens, list_k(p), p->num_heads_q, p->head_dim_v, target,
+                                    p->scenario, p->ori_win_left, p->kv_dtype == SAS_DT_FP8E4M3).total;
+  return SAS_OK;
 }
 
 int sas_backward_workspace_size(const sas_params_t* p, size_t* bytes) {

@@ -210,8 +210,10 @@ SAS_HD static inline SasBwdLayout sas_bwd_layout(size_t fwd_total, int64_t T, in
 }
 
 // ---- kernel parameter blocks (passed by value) ----
+// cu_ends (here and in the resolution's arguments): act_q holds the sequences' cumulative
+// ends (q_prefix's successors), not their lengths.
 struct SasPlanArgs {
-  int32_t T, B, scenario, win_left, cmp_ratio, K, H, target;
+  int32_t T, B, scenario, win_left, cmp_ratio, K, H, target, cu_ends;
 };
 
 struct SasFwdArgs {

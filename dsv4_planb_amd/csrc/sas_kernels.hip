@@ -60,7 +60,7 @@ __device__ TokInfo token_info(const SasPlanArgs& a, const int* q_prefix, const i
   }
   if (b < 0) return ti;
   int s = t - q_prefix[b];
-  int aq = act_q[b];
+  int aq = act_q[b] - (a.cu_ends ? q_prefix[b] : 0);
   ti.sg = b;
   if (s >= aq) return ti;
   int sg = seqused_kv[b] - aq + s;                    // golden.py:125
@@ -401,6 +401,7 @@ struct RsShared {
 struct SasResolveArgs {
   const int* q_prefix;    // the call's lengths (per batch)
   const int* act_q;
+  int cu_ends;            // act_q holds cumulative ends
   const int* seqused_kv;
   const int* ori_bt;
   const int* idx;
@@ -466,14 +467,14 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
     // unowned when the plan was built: refused if the call's lengths give the token
     // to the candidate batch (sg_plan)
     if (b < 0 && sg_plan >= 0 && sg_plan < a.B) {
-      const int q0 = r.q_prefix[sg_plan], nq = r.act_q[sg_plan];
+      const int q0 = r.q_prefix[sg_plan], nq = r.act_q[sg_plan] - (r.cu_ends ? q0 : 0);
       if (q0 <= t && t - q0 < nq) nwin_live = -1;
     }
     return 0;
   }
   // The batch's live lengths, issued before (and so landing with) the block-table
   // loads below, which start at the plan's window.
-  const int q0 = r.q_prefix[b], nq = r.act_q[b], kv_live = r.seqused_kv[b];
+  const int q0 = r.q_prefix[b], nq = r.act_q[b] - (r.cu_ends ? q0 : 0), kv_live = r.seqused_kv[b];
   int* out = r.rows ? r.rows + (size_t)t * a.list_stride : nullptr;
   uint64_t* aout = r.addr + (size_t)t * a.list_stride;
   // fp8 KV: each row's dequantisation scale s and 1 / s beside its address (a -1

@@ -234,12 +234,21 @@ def sparse_attn_sharedkv_metadata(
     if layout_q == "TND":
         if cu_seqlens_q is None:
             raise ValueError("cu_seqlens_q is required for TND")
-        cu = cu_seqlens_q.to(dev, torch.int32)
         cu_host = cu_seqlens_q.detach().to("cpu", torch.int64)  # (the plan's record)
-        batch = cu.numel() - 1
-        total = int(cu_host[-1].item())  # the token count sizes the plan
-        q_prefix, act_q = cu[:-1], cu[1:] - cu[:-1]
+        batch = cu_host.numel() - 1
+        total = int(cu_host[-1])  # the token count sizes the plan
         qp_host, aq_host = cu_host[:-1], cu_host[1:] - cu_host[:-1]
+        if cu_seqlens_q.device.type == "cpu" and not torch.cuda.is_current_stream_capturing():
+            # both on the device by one copy from pinned memory, which the host does not
+            # wait for (the allocator keeps the block until the stream has read it)
+            host = torch.empty(2 * batch, dtype=torch.int32, pin_memory=True)
+            host[:batch] = qp_host
+            host[batch:] = aq_host
+            lens = host.to(dev, non_blocking=True)
+            q_prefix, act_q = lens[:batch], lens[batch:]
+        else:
+            cu = cu_seqlens_q.to(dev, torch.int32)
+            q_prefix, act_q = cu[:-1], cu[1:] - cu[:-1]
     else:
         batch = batch_size if batch_size > 0 else seqused_kv.numel()
         total = batch * max_seqlen_q

@@ -119,6 +119,9 @@ int sas_workspace_size(const sas_params_t* p, size_t* bytes);
 int sas_plan_size(const sas_params_t* p, size_t* n_int32);
 /* Target number of work units (num_cus * units_per_cu after defaults). */
 int sas_target_units(const sas_params_t* p, int32_t* units);
+/* Validation and a call's three sizes at once: sizes[0] the work units the plan
+ * balances for, sizes[1] the plan's int32 entries, sizes[2] the workspace bytes. */
+int sas_call_sizes(const sas_params_t* p, int64_t* sizes /* [3] */);
 
 /* ---- device entry points (asynchronous on stream) ---- */
 /* Split-KV scheduler: per-token row spans and work units balanced over CUs,
@@ -146,6 +149,12 @@ int sas_plan(const sas_params_t* p, const int32_t* q_prefix, const int32_t* act_
  * instead of SAS_OK. */
 int sas_forward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan,
                 void* workspace, size_t workspace_bytes, sas_stream_t stream);
+/* sas_forward with t->act_q_lens holding each sequence's cumulative end (the
+ * successor of its q_prefix entry: cu_seqlens_q + 1 where q_prefix is cu_seqlens_q)
+ * instead of its length, so that a caller with cu_seqlens_q on the device launches
+ * nothing to form the lengths. */
+int sas_forward_cu(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan,
+                   void* workspace, size_t workspace_bytes, sas_stream_t stream);
 /* The stages of sas_forward, for timing and debugging (same workspace).
  * sas_resolve writes every token's row lists (codes too) and counts; sas_attend
  * launches the attention dispatch exactly as sas_forward does (where the forward
