@@ -186,10 +186,12 @@ SAS_HD static inline SasBwdLayout sas_bwd_layout(size_t fwd_total, int64_t T, in
   L.chunk_tokens = (int)(T > 0 ? T : 1);
   L.item_cap = 0;
   if (!L.tile) return L;
-  int64_t chunk = (int64_t)(SAS_BWD_SPILL_BYTES / per_token);
-  if (chunk < 1) chunk = 1;
-  const int64_t runs = (T + chunk - 1) / chunk;
-  chunk = ((T + runs - 1) / runs + 63) / 64 * 64;
+  // (at least one: per_token is within the bound); the runs are of about equal length, in
+  // whole groups of 64 tokens where the bound leaves room for that
+  const int64_t most = (int64_t)(SAS_BWD_SPILL_BYTES / per_token);
+  const int64_t runs = (T + most - 1) / most;
+  int64_t chunk = ((T + runs - 1) / runs + 63) / 64 * 64;
+  if (chunk > most) chunk = most;
   if (chunk > T) chunk = T;
   L.chunk_tokens = (int)chunk;
   // groups of a run: at most chunk / group + one partial group per sequence; tiles of a
