@@ -16,9 +16,8 @@
 //                     16x16x32 MFMAs (K rows from LDS, Q^T and dO^T fragments in
 //                     registers), P and dS in registers, then dq^T += K^T dS^T
 //                     (K^T read transposed from the same row-major tile, dS^T
-//                     straight from the accumulator layout).  Two tile buffers: the
-//                     next tile's rows are loaded into registers during this one's
-//                     MFMAs and stored after them.
+//                     straight from the accumulator layout).  Three tile buffers,
+//                     filled by LDS-direct DMA, one barrier per tile.
 //   bwd_dkv_kernel    the KV pools' gradient (dK from dS and q, dV from P and
 //                     dO): one workgroup per work unit, the tile's gradient summed
 //                     over all heads in registers, then fp32 atomics into
@@ -67,6 +66,18 @@ __device__ __forceinline__ bw_f32x4 bw_mfma(const u32x4_t& a, const u32x4_t& b, 
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(bw_f16x8, a),
                                                   __builtin_bit_cast(bw_f16x8, b), c, 0, 0, 0);
+}
+
+// acc + the two 16-bit values of v, each times zero: acc, or a NaN where one is not finite.
+template <int QT>
+__device__ __forceinline__ float dot2_zero(uint32_t v, uint32_t zero, float acc) {
+  if constexpr (QT == 0) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, v), __builtin_bit_cast(b2, zero), acc, false);
+  } else {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, v), __builtin_bit_cast(h2, zero), acc, false);
+  }
 }
 
 // D = <dO, out> (less dlse when the LSE has a gradient) and the sink term
@@ -144,83 +155,117 @@ struct SasBwdSpill {
   int* flags;
 };
 
+// A tile's LDS layout: latent rows at a 1088-B stride, 16-B chunk c of row r at c ^ f(r), f
+// = 2 (r bit 2) + (r bit 3); rope rows of 128 B, chunk c at c ^ fr(r), fr the three bits of
+// (r >> 1) & 7 rotated left by one.  The b128 reads (16 rows, one chunk) and the
+// transposed ones (rows 4 g .. 4 g + 3 and 4 g + 4 .. 4 g + 7 x 32 B per 32 lanes) then
+// touch every bank once per 256 B.
+template <int DQK, bool SPILL>
+struct DqLds {
+  static constexpr int STRA = 1024 + 64, ROWR = (DQK - 512) * 2;
+  static constexpr int TILEA = BW_TILE * STRA, TILEB = TILEA + BW_TILE * ROWR;
+  __attribute__((aligned(16))) uint8_t tiles[3 * TILEB];
+  // SPILL: a wave's P and dS of a tile, [16 heads][32 keys] each, for the transpose
+  __attribute__((aligned(16))) uint8_t tp[SPILL ? 4 * 2048 : 16];
+};
+
+// Ring of three tiles: tile i is computed while tile i + 1 arrives and tile i + 2's DMAs
+// (wave w: rows 8 w .. + 7, 8 latent and one rope instruction) are issued between the
+// S / dP chain's MFMAs; one barrier per tile.  What bounds it is the S / dP chain (36
+// k-steps, one LDS read and two dependent MFMAs each, on the SIMD's only wave: q, dO and
+// dq^T fill its registers).  Before, the next tile's rows went through registers and a
+// second barrier, the first tile was fetched after the query's rows, and the check for
+// infinities and NaNs took four instructions per value.  Measured, with the spill: 4 documents
+// of 608 .. 1,697 tokens, 128 heads, top-k 512, 1,390 -> 1,070 us; documents of 1,082
+// and 971 tokens, 64 heads, window only, d_qk 512, 232 -> 185 us.
 template <int DQK, int QT, bool SPILL>
-__global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint16_t* __restrict__ q,
-                                                        const uint16_t* __restrict__ dout,
-                                                        const uint64_t* __restrict__ addr_list,
-                                                        const int2* __restrict__ tok,
-                                                        const float* __restrict__ lse,
-                                                        const float* __restrict__ dterm,
-                                                        const int* __restrict__ plan,
-                                                        float* __restrict__ dq, SasBwdSpill sp) {
+__device__ __forceinline__ void dq_unit(DqLds<DQK, SPILL>& sm, const int4 ur, int hg, const SasFwdArgs& a,
+                                        const uint16_t* __restrict__ q, const uint16_t* __restrict__ dout,
+                                        const uint64_t* __restrict__ addr_list,
+                                        const int2* __restrict__ tok, const float* __restrict__ lse,
+                                        const float* __restrict__ dterm, const int* __restrict__ plan,
+                                        float* __restrict__ dq, const SasBwdSpill& sp) {
   constexpr int DV = 512;
+  constexpr bool ROPE = DQK > DV;
   constexpr int KS = DQK / 32;         // k-steps of S^T = K Q^T (18 / 16)
   constexpr int VKS = DV / 32;         // k-steps of dP^T = V dO^T (16)
   constexpr int NDB = DQK / 16;        // 16-dimension blocks of dq^T (36 / 32)
-  constexpr int CH = DQK / 8;          // 16-B chunks per row
-  constexpr int KSTR = DQK * 2 + 16;   // row-major tile: row stride in bytes
-  constexpr int NLD = (BW_TILE * CH + 255) / 256;  // chunks per thread and tile (9 / 8)
-  // two tiles: the one computed on and the next one, stored from registers after
-  // the MFMAs of this one
-  __shared__ __attribute__((aligned(16))) uint8_t kt[2][BW_TILE * KSTR];
-  // SPILL: a wave's P and dS of a tile, [16 heads][32 keys] each, for the transpose
-  __shared__ __attribute__((aligned(16))) uint8_t tp[SPILL ? 4 * 2048 : 16];
+  constexpr int STRA = DqLds<DQK, SPILL>::STRA, ROWR = DqLds<DQK, SPILL>::ROWR;
+  constexpr int TILEA = DqLds<DQK, SPILL>::TILEA, TILEB = DqLds<DQK, SPILL>::TILEB;
+  constexpr int CPT = ROPE ? 9 : 8;    // DMA instructions per wave and tile
+  typedef __attribute__((address_space(3))) uint8_t l_u8;
+  typedef __attribute__((address_space(3))) void l_void;
+  typedef short tr_s4 __attribute__((ext_vector_type(4)));
+  l_u8* const lds = (l_u8*)sm.tiles;
 
-  const int HG = (a.H + BW_HEADS - 1) / BW_HEADS;
-  const int u = blockIdx.x / HG, hg = blockIdx.x - u * HG;
-  if (!plan_matches(plan, a) || u >= plan[PH_UNITS]) return;  // refused plan: prep zeroed dq
-  const int* ur = plan + SAS_PLAN_HDR + (size_t)SAS_TOK_W * a.T + (size_t)u * SAS_UNIT_W;
-  const int t = ur[0], split = ur[3];
-  if (SPILL && (t < sp.t0 || t >= sp.t1)) return;  // a token of another run
+  const int t = ur.x, split = ur.w;
   if (split < 0) return;  // a q row no batch owns: zero (bwd_prep_kernel)
-  const int* tk = plan + SAS_PLAN_HDR + (size_t)t * SAS_TOK_W;
-  const int splits = tk[TK_SPLITS];
-  const int2 tr = tok[t];  // row counts at the call's lengths (the resolver's)
-  if (tr.x < 0) return;    // refused token: zero (bwd_prep_kernel)
-  const int r0 = ur[1];
-  const int r1 = min(split == splits - 1 ? tr.x + tr.y : min(ur[2], tr.x + tr.y), a.list_stride);
-  const int ntiles = r1 > r0 ? (r1 - r0 + BW_TILE - 1) / BW_TILE : 0;
-  const uint64_t* alist = addr_list + (size_t)t * a.list_stride;
-
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  if (SPILL && (t < sp.t0 || t >= sp.t1)) return;  // a token of another run
+  const int r0 = ur.y;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, g = lane >> 4;
   const int h = hg * BW_HEADS + w * 16 + n16;
   const bool hvalid = h < a.H;
   const int hc = min(h, a.H - 1);
   const size_t th = (size_t)t * a.H + hc;
+  // a tile's row addresses of this wave: lane l holds row 8 w + (l & 7)
+  const uint64_t* alist = addr_list + (size_t)t * a.list_stride;
+  typedef __attribute__((address_space(1))) const uint64_t g_u64;
+  auto addrs = [&](int i) -> uint64_t {
+    return ((g_u64*)(uintptr_t)alist)[min(r0 + i * BW_TILE + 8 * w + (lane & 7), a.list_stride - 1)];
+  };
+  uint64_t av = addrs(0), av1 = addrs(1), av2 = addrs(2);
+  const int* tk = plan + SAS_PLAN_HDR + (size_t)t * SAS_TOK_W;
+  const int splits = tk[TK_SPLITS];
+  const int2 tr = tok[t];  // row counts at the call's lengths (the resolver's)
+  if (tr.x < 0) return;    // refused token: zero (bwd_prep_kernel)
+  const int r1 = min(split == splits - 1 ? tr.x + tr.y : min(ur.z, tr.x + tr.y), a.list_stride);
+  const int ntiles = r1 > r0 ? (r1 - r0 + BW_TILE - 1) / BW_TILE : 0;
 
-  // A tile's rows: chunk ch = tid + 256 c (row ch / CH, 16-B chunk ch % CH).  The
-  // row addresses of tile i + 2 and the chunks of tile i + 1 are loaded while tile i
-  // is computed; rows past the unit's end (address 0) are zeros.
-  uint64_t ra[NLD];
-  u32x4_t pre[NLD];
-  auto addrs = [&](int i) {
-    const int rb = r0 + i * BW_TILE;
-#pragma unroll
-    for (int c = 0; c < NLD; ++c) {
-      const int ch = tid + 256 * c, row = ch / CH;
-      ra[c] = ch < BW_TILE * CH && rb + row < r1 ? alist[rb + row] : 0;
+  // row 8 w + k: lane l fetches latent chunk l ^ f, f = 2 (k >> 2) + (w & 1); rope: lane 8 k +
+  // j fetches chunk j ^ fr of row 8 w + k
+  const uint32_t vlat = 16u * ((uint32_t)lane ^ (uint32_t)(w & 1));
+  const uint32_t rx = (uint32_t)((8 * w + (lane >> 3)) >> 1) & 7u;
+  const uint32_t vrope = 1024u + 16u * (((uint32_t)lane & 7u) ^ (((rx & 3u) << 1) | (rx >> 2)));
+  auto tail = [&](uint64_t v, int i) -> uint64_t {  // rows past r1 read the zero row
+    return r0 + i * BW_TILE + 8 * w + (lane & 7) < r1 ? v : (uint64_t)g_zero_row;
+  };
+  auto dma_lat = [&](int sl, uint64_t v, int k) {
+    const uint64_t ra = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), k) << 32) |
+                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, k);
+    uint32_t vo = vlat;
+    if (k >= 4) {  // (formed here rather than kept across the loop)
+      asm volatile("" : "+v"(vo));
+      vo ^= 32u;
+    }
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        __builtin_amdgcn_make_buffer_rsrc((void*)ra, (short)0, 1024, 0x00020000),
+        (l_void*)(lds + sl * TILEB + (8 * w + k) * STRA), 16, vo, 0, 0, 0);
+  };
+  // (in assembly: the compiler takes a global LDS-direct load for a FLAT access and then
+  // drains both counters at the next wait of either)
+  auto dma_rope = [&](int sl, uint64_t v) {
+    if constexpr (ROPE) {
+      const int from = lane >> 3;
+      const uint64_t src = (((uint64_t)(uint32_t)__shfl((int)(v >> 32), from) << 32) |
+                            (uint32_t)__shfl((int)(uint32_t)v, from)) + vrope;
+      const uint32_t m0 = (uint32_t)(uintptr_t)(lds + sl * TILEB + TILEA + 8 * w * ROWR);
+      uint32_t keep;  // the compiler's own value of m0
+      asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+                   "s_mov_b32 m0, %0" : "=&s"(keep) : "v"(src), "s"(m0) : "memory");
     }
   };
-  auto fetch = [&]() {
+  // tiles 0 and 1 (dead tiles too), ahead of the query's loads
+  av = tail(av, 0);
+  av1 = tail(av1, 1);
 #pragma unroll
-    for (int c = 0; c < NLD; ++c) {
-      const int ch = tid + 256 * c, cc = ch - (ch / CH) * CH;
-      pre[c] = ra[c] ? gload16(ra[c] + 16 * cc) : u32x4_t{0, 0, 0, 0};
-    }
-  };
-  auto stash = [&](int buf) {
+  for (int k = 0; k < 8; ++k) dma_lat(0, av, k);
+  dma_rope(0, av);
 #pragma unroll
-    for (int c = 0; c < NLD; ++c) {
-      const int ch = tid + 256 * c, row = ch / CH, cc = ch - row * CH;
-      if (ch < BW_TILE * CH) *reinterpret_cast<u32x4_t*>(kt[buf] + row * KSTR + cc * 16) = pre[c];
-    }
-  };
-  if (ntiles > 0) {
-    addrs(0);
-    fetch();
-    if (ntiles > 1) addrs(1);
-  }
+  for (int k = 0; k < 8; ++k) dma_lat(1, av1, k);
+  dma_rope(1, av1);
+  asm volatile("" ::: "memory");
 
   u32x4_t qf[KS], of[VKS];
   {
@@ -235,19 +280,19 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
   const float c = a.scale_log2;
   const float scale = c * 0.6931471805599453f;
   if constexpr (SPILL) {
-    // an infinity or a NaN: all exponent bits set (both halves of each dword)
-    constexpr uint32_t EXP = QT == 0 ? 0x7f80u : 0x7c00u;
-    bool bad = false;
-    auto check = [&](const u32x4_t& v) {
+    // an infinity or a NaN times zero is a NaN: one dot product with zeros per two values
+    uint32_t zero = 0;
+    asm volatile("" : "+v"(zero));  // (opaque: the products are not folded)
+    float z = 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        bad = bad || (v[e] & EXP) == EXP || ((v[e] >> 16) & EXP) == EXP;
-    };
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) check(qf[ks]);
+      for (int e = 0; e < 4; ++e) z = dot2_zero<QT>(qf[ks][e], zero, z);
 #pragma unroll
-    for (int ks = 0; ks < VKS; ++ks) check(of[ks]);
-    if (__any(bad) && lane == 0) {
+    for (int ks = 0; ks < VKS; ++ks)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z = dot2_zero<QT>(of[ks][e], zero, z);
+    if (__any(z != 0.f) && lane == 0) {
       sp.flags[1 + t] = 1;
       atomicAdd(sp.flags, 1);
     }
@@ -257,25 +302,44 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
   // position 8 g + 4 kb + r), and ds_read_b64_tr_b16 returns 4 heads (4 g .. + 3) of
   // one position per lane, stored as 8 B of its key's record.  The 32-B halves of a row
   // are swapped for heads 4 .. 7 and 12 .. 15, so that the transposed reads touch every
-  // bank once per 256 B.
-  uint8_t* const tpw = tp + (SPILL ? w * 2048 : 0);
-  const bool sp_wave = SPILL && hg * BW_HEADS + w * 16 < sp.row_bytes / 4;  // a padded head chunk ends
-  uint8_t* sp_row = nullptr;
-  if constexpr (SPILL)
-    sp_row = sp.data + (1 + (size_t)(t - sp.t0) * sp.stride) * sp.row_bytes +
-             (2 * hg + (w >> 1)) * 128 + (16 * (w & 1) + 4 * g) * 2;
+  // bank once per 256 B.  Every wave makes the same four stores in every tile (positions
+  // past the end, and waves past the padded heads, at an offset past the buffer, which
+  // drops them), so that the waits for the ring's DMAs can count them.
+  l_u8* const tpw = (l_u8*)sm.tp + (SPILL ? w * 2048 : 0);
+  const bool sp_wave = SPILL && hg * BW_HEADS + w * 16 < sp.row_bytes / 4;  // (a padded head chunk ends)
+  const auto sp_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(SPILL ? sp.data : nullptr), (short)0,
+      (int)((1u + (uint32_t)(sp.t1 - sp.t0) * (uint32_t)sp.stride) * (uint32_t)sp.row_bytes), 0x00020000);
+  const uint32_t sp_off = (1u + (uint32_t)(t - sp.t0) * (uint32_t)sp.stride) * (uint32_t)sp.row_bytes +
+                          (uint32_t)((2 * hg + (w >> 1)) * 128 + (16 * (w & 1) + 4 * g) * 2);
   bw_f32x4 acc[NDB];
 #pragma unroll
   for (int i = 0; i < NDB; ++i) acc[i] = bw_f32x4{0.f, 0.f, 0.f, 0.f};
-  if (ntiles > 0) stash(0);
-  __syncthreads();
 
-  typedef short tr_s4 __attribute__((ext_vector_type(4)));
+  // K fragments: row 16 kb + n16, chunk 4 ks + g; K^T fragments: rows 4 g + (n16 >> 2) (+ 16),
+  // dimensions 16 db + 4 (n16 & 3) .. + 3
+  const uint32_t kf0 = n16 * STRA + 16 * (g ^ (2 * ((n16 >> 2) & 1) + ((n16 >> 3) & 1)));
+  const uint32_t kx = (uint32_t)(n16 >> 1) & 7u;
+  const uint32_t kfr = TILEA + n16 * ROWR + 16 * (g ^ (int)(((kx & 3u) << 1) | (kx >> 2)));
+  const int trow = 4 * g + (n16 >> 2);
+  const uint32_t tb0 = trow * STRA + 32 * (g & 1) + 16 * (((n16 >> 1) & 1) ^ ((g >> 1) & 1)) + 8 * (n16 & 1);
+  const uint32_t tx = (uint32_t)(trow >> 1) & 7u;
+  const uint32_t tbr = TILEA + trow * ROWR + 16 * (((n16 >> 1) & 1) ^ (int)(((tx & 3u) << 1) | (tx >> 2))) + 8 * (n16 & 1);
+
+  int sl = 0;
   for (int i = 0; i < ntiles; ++i) {
     const int rb = r0 + i * BW_TILE;
-    const uint8_t* tl = kt[i & 1];
-    if (i + 1 < ntiles) fetch();
-    if (i + 2 < ntiles) addrs(i + 2);
+    // Tile i has landed: younger are tile i + 1's DMAs, an address load and, from the
+    // second tile on, the last tile's stores (in the first, the query's loads)
+    if (i == 0)
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+    else
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(CPT + 1 + (SPILL ? 4 : 0), 0));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const l_u8* tl = lds + sl * TILEB;
+    const int s2 = sl == 0 ? 2 : sl - 1;  // tile i + 2's slot: tile i - 1's
+    const uint64_t vn = tail(av2, i + 2);
     // S^T and dP^T: two blocks of 16 keys each, one chain of 2 KS steps (block
     // kb = st / KS, k-step st % KS).  The K fragments are read BW_AHEAD steps ahead
     // (an LDS read takes several MFMAs' time to return, and this wave is the
@@ -289,7 +353,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
     {
       auto kfrag = [&](int st) -> u32x4_t {
         const int kb = st / KS, ks = st - kb * KS;
-        return *reinterpret_cast<const u32x4_t*>(tl + (16 * kb + n16) * KSTR + 16 * g + 64 * ks);
+        return ks < 16 ? lds_read_b128(tl + kf0 + 16 * STRA * kb + 64 * ks)
+                       : lds_read_b128(tl + ((kfr + 16 * ROWR * kb) ^ (64u * (uint32_t)(ks - 16))));
       };
       u32x4_t kf[BW_AHEAD + 1];
 #pragma unroll
@@ -299,12 +364,15 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
       for (int st = 0; st < 2 * KS; ++st) {
         if (st + BW_AHEAD < 2 * KS) kf[(st + BW_AHEAD) % (BW_AHEAD + 1)] = kfrag(st + BW_AHEAD);
         const int kb = st / KS, ks = st - kb * KS;
-        const u32x4_t av = kf[st % (BW_AHEAD + 1)];
-        s[kb] = bw_mfma<QT>(av, qf[ks], s[kb]);
-        if (ks < VKS) dp[kb] = bw_mfma<QT>(av, of[ks], dp[kb]);
+        const u32x4_t av_ = kf[st % (BW_AHEAD + 1)];
+        s[kb] = bw_mfma<QT>(av_, qf[ks], s[kb]);
+        if (ks < VKS) dp[kb] = bw_mfma<QT>(av_, of[ks], dp[kb]);
+        if ((st & 3) == 1 && (st >> 2) < 8) dma_lat(s2, vn, st >> 2);
         BW_SB();
       }
+      dma_rope(s2, vn);
     }
+    av2 = addrs(i + 3);
     // P = e^(s - lse) and dS = P (dP - D) for keys 16 kb + 4 g + r of head n16
     float ds[8], pr[8];
 #pragma unroll
@@ -320,7 +388,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
 #pragma unroll
     for (int e = 0; e < 4; ++e) bds[e] = pack2_q16<QT>(ds[2 * e], ds[2 * e + 1]);
     if constexpr (SPILL) {
-      if (sp_wave) {
+      {
         u32x4_t xs, xp;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {  // (heads at or past H: zeros)
@@ -328,9 +396,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
           xp[e] = hvalid ? pack2_q16<QT>(pr[2 * e], pr[2 * e + 1]) : 0u;
         }
         const int wo = 64 * n16 + 16 * (g ^ (2 * ((n16 >> 2) & 1)));
-        *reinterpret_cast<u32x4_t*>(tpw + wo) = xs;
-        *reinterpret_cast<u32x4_t*>(tpw + 1024 + wo) = xp;
-        const uint8_t* ro = tpw + 64 * (4 * g + (n16 >> 2)) + 8 * (n16 & 3);
+        *reinterpret_cast<__attribute__((address_space(3))) u32x4_t*>(tpw + wo) = xs;
+        *reinterpret_cast<__attribute__((address_space(3))) u32x4_t*>(tpw + 1024 + wo) = xp;
+        const l_u8* ro = tpw + 64 * (4 * g + (n16 >> 2)) + 8 * (n16 & 3);
         tr_s4 v[2][2];
 #pragma unroll
         for (int x = 0; x < 2; ++x)
@@ -341,12 +409,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
           const int p = rb + 16 * ((n16 >> 2) & 1) + 4 * (2 * x + (n16 >> 3)) + (n16 & 3);
-          if (p < r1 && p < sp.stride) {
-            typedef __attribute__((address_space(1))) tr_s4 g_s4;
-            uint8_t* dst = sp_row + (size_t)p * sp.row_bytes;
-            *(g_s4*)(uintptr_t)dst = v[x][0];
-            *(g_s4*)(uintptr_t)(dst + 64) = v[x][1];
-          }
+          const uint32_t off = sp_wave && p < r1 && p < sp.stride ? sp_off + (uint32_t)p * (uint32_t)sp.row_bytes : ~0u - 127u;
+          typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v[x][0]), sp_rsrc, off, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v[x][1]), sp_rsrc, off + 64u, 0, 0);
         }
       }
     }
@@ -355,14 +421,14 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
     // ds_read_b64_tr_b16 gives lane j element j & 3 of the 8 bytes lane (j >> 2) + 4 e
     // addresses, for e = 0 .. 3; so lane i of block g addresses key 4 g + (i >> 2)
     // (+ 16), dimensions 16 db + 4 (i & 3) .. + 3.
-    const uint8_t* ta = tl + (4 * g + (n16 >> 2)) * KSTR + 8 * (n16 & 3);
     {
       // the K^T fragments, read BW_AHEAD_T blocks ahead
       auto kt_frag = [&](int db) -> u32x4_t {
-        const tr_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) tr_s4*)(ta + 32 * db));
-        const tr_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) tr_s4*)(ta + 16 * KSTR + 32 * db));
+        const l_u8* p = db < 32 ? tl + (tb0 ^ (32u * (uint32_t)(db & 1))) + 64 * (db >> 1)
+                                : tl + (tbr ^ (32u * (uint32_t)(db - 32)));
+        const int up = db < 32 ? 16 * STRA : 16 * ROWR;
+        const tr_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) tr_s4*)p);
+        const tr_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) tr_s4*)(p + up));
         return u32x4_t{(uint32_t)(uint16_t)lo[0] | ((uint32_t)(uint16_t)lo[1] << 16),
                        (uint32_t)(uint16_t)lo[2] | ((uint32_t)(uint16_t)lo[3] << 16),
                        (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16),
@@ -379,9 +445,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
         BW_SB();
       }
     }
-    if (i + 1 < ntiles) stash((i + 1) & 1);
-    __syncthreads();  // tile i + 1 stored; every wave is done with tile i
+    sl = sl == 2 ? 0 : sl + 1;
   }
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));  // the dead tiles' DMAs have landed
   if (!hvalid) return;
   // lane holds dimensions 16 db + 4 g .. + 3 of head h
   float* dqr = dq + ((size_t)t * a.H + h) * DQK + 4 * g;
@@ -398,6 +464,28 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
       *reinterpret_cast<float4*>(dqr + 16 * db) = v;
     }
   }
+}
+
+template <int DQK, int QT, bool SPILL>
+__global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint16_t* __restrict__ q,
+                                                        const uint16_t* __restrict__ dout,
+                                                        const uint64_t* __restrict__ addr_list,
+                                                        const int2* __restrict__ tok,
+                                                        const float* __restrict__ lse,
+                                                        const float* __restrict__ dterm,
+                                                        const int* __restrict__ plan,
+                                                        float* __restrict__ dq, SasBwdSpill sp) {
+  __shared__ DqLds<DQK, SPILL> sm;
+  const int HG = (a.H + BW_HEADS - 1) / BW_HEADS;
+  const int u = blockIdx.x / HG, hg = blockIdx.x - u * HG;
+  // (the unit's record with the plan's header: one memory round trip for both)
+  const int* up = plan + SAS_PLAN_HDR + (size_t)SAS_TOK_W * a.T + (size_t)u * SAS_UNIT_W;
+  int4 ur = make_int4(up[0], up[1], up[2], up[3]);
+  const int units = plan[PH_UNITS];
+  const bool ok = plan_matches(plan, a);
+  asm volatile("" : "+s"(ur.x), "+s"(ur.y), "+s"(ur.z), "+s"(ur.w));
+  if (!ok || u >= units) return;  // refused plan: prep zeroed dq
+  dq_unit<DQK, QT, SPILL>(sm, ur, hg, a, q, dout, addr_list, tok, lse, dterm, plan, dq, sp);
 }
 
 // ---------------------------------------------------------------------------
