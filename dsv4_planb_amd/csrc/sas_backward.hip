@@ -8,11 +8,11 @@
 //   dsink = -sum_t e^(sink - lse) D
 // over the same row lists the forward attends (the resolver's output).
 //
-//   bwd_prep_kernel   D and the sink term per (token, head); zeroes the dq rows
-//                     that are accumulated by several units (split tokens) or
-//                     that no batch owns.
+//   bwd_prep_kernel   zeroes the dq rows that are accumulated by several units (split
+//                     tokens) or that no batch owns.
 //   bwd_dq_kernel     one workgroup per (work unit, 64 heads): each wave owns 16
-//                     heads.  Per 32-row tile: S^T = K Q^T and dP^T = V dO^T as
+//                     heads.  D and the sink term per (token, head); then, per 32-row
+//                     tile: S^T = K Q^T and dP^T = V dO^T as
 //                     16x16x32 MFMAs (K rows from LDS, Q^T and dO^T fragments in
 //                     registers), P and dS in registers, then dq^T += K^T dS^T
 //                     (K^T read transposed from the same row-major tile, dS^T
@@ -80,67 +80,49 @@ __device__ __forceinline__ float dot2_zero(uint32_t v, uint32_t zero, float acc)
   }
 }
 
-// D = <dO, out> (less dlse when the LSE has a gradient) and the sink term
-// -e^(sink - lse) D, one wave per (token, head): workgroup x takes token x / HB and
-// heads 4 (x % HB) .. + 3, HB = ceil(H / 4) (lane l covers dimensions 8 l .. 8 l + 7
-// of d_v = 512).  One wave per head keeps every head's loads in flight at once; a
-// wave walking a token's heads in turn waits for each head's rows before the next.
-template <int QT>
-__global__ __launch_bounds__(256) void bwd_prep_kernel(SasFwdArgs a, int dqk,
-                                                       const int* __restrict__ plan,
+// What the dq kernel leaves out, per (token, BP_HEADS heads): the terms of tokens that no
+// batch owns (or whose plan is refused), and the zeros of their dq rows and of those that
+// several units add to; and the flags of a call whose P and dS are spilled (else null).
+constexpr int BP_HEADS = 64;
+__global__ __launch_bounds__(256) void bwd_prep_kernel(SasFwdArgs a, int dqk, const int* __restrict__ plan,
                                                        const int2* __restrict__ tok,
-                                                       const uint16_t* __restrict__ dout,
-                                                       const uint16_t* __restrict__ out,
-                                                       const float* __restrict__ lse,
-                                                       const float* __restrict__ dlse,
-                                                       const float* __restrict__ sinks,
-                                                       float* __restrict__ dterm,
-                                                       float* __restrict__ sterm,
-                                                       float* __restrict__ dq,
-                                                       int* __restrict__ flags) {
-  constexpr int DV = 512;
-  const int HB = (a.H + 3) / 4;
-  const int t = blockIdx.x / HB, h = (blockIdx.x - t * HB) * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (flags && threadIdx.x == 0 && blockIdx.x == t * HB) {
+                                                       float* __restrict__ dterm, float* __restrict__ sterm,
+                                                       float* __restrict__ dq, int* __restrict__ flags) {
+  const int HB = (a.H + BP_HEADS - 1) / BP_HEADS;
+  const int t = blockIdx.x / HB, h0 = (blockIdx.x - t * HB) * BP_HEADS;
+  const int tid = threadIdx.x, nh = min(BP_HEADS, a.H - h0);
+  if (flags && tid == 0 && h0 == 0) {
     flags[1 + t] = 0;
     if (t == 0) flags[0] = 0;
   }
-  if (h >= a.H) return;
   const bool ok = plan_matches(plan, a);
   const int* tk = plan + SAS_PLAN_HDR + (size_t)t * SAS_TOK_W;
   const int b = ok ? tk[TK_B] : -1;
   // (a token the resolver refused for a stale plan counts as unowned)
   const bool owned = b >= 0 && b < a.B && tok[t].x >= 0;
-  const bool zero_dq = !owned || tk[TK_SPLITS] > 1;
-  {
-    const size_t th = (size_t)t * a.H + h;
-    float d = 0.f;
-    if (owned) {
-      const u32x4_t go = reinterpret_cast<const u32x4_t*>(dout + th * DV)[lane];
-      const u32x4_t oo = reinterpret_cast<const u32x4_t*>(out + th * DV)[lane];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        d = fmaf(q16_to_f32<QT>(go[e] & 0xffffu), q16_to_f32<QT>(oo[e] & 0xffffu), d);
-        d = fmaf(q16_to_f32<QT>(go[e] >> 16), q16_to_f32<QT>(oo[e] >> 16), d);
-      }
-      d = wave_sum(d);
-      // a gradient of the LSE: d lse / d s_j = P_j and d lse / d sink = P_sink, so it
-      // enters as dS = P (dP - (D - dlse)) and dsink = -P_sink (D - dlse)
-      if (dlse) d -= dlse[th];
-    }
-    if (lane == 0) {
-      dterm[th] = d;
-      const float s = sinks[h];
-      // a sink of -inf has P_sink = 0 (lse may be -inf too when nothing is attended)
-      sterm[th] = (!owned || s == -INFINITY || d == 0.f) ? 0.f : -__expf(s - lse[th]) * d;
-    }
-    if (zero_dq) {
-      float4* row = reinterpret_cast<float4*>(dq + th * dqk);
-      for (int i = lane; i < dqk / 4; i += 64) row[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+  const size_t th = (size_t)t * a.H + h0;
+  if (!owned && tid < nh) {
+    dterm[th + tid] = 0.f;
+    sterm[th + tid] = 0.f;
+  }
+  if (!owned || tk[TK_SPLITS] > 1) {
+    float4* row = reinterpret_cast<float4*>(dq + th * dqk);
+    for (int i = tid; i < nh * dqk / 4; i += 256) row[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 }
+
+// D = <dO, out> (less dlse when the LSE has a gradient) and the sink term -e^(sink - lse) D,
+// which the dq kernel computes where it holds the dO rows and writes for the kernels after
+// it: a kernel of its own reads dO once more and was bound by that (4 documents of 608 ..
+// 1,697 tokens, 128 heads: 221 us; now 8 us for bwd_prep_kernel and 100 us more in the dq
+// kernel; documents of 1,082 and 971 tokens, 64 heads: 59 us, now 6 and 25).
+struct SasBwdTerms {
+  const uint16_t* out;
+  const float* dlse;  // or null
+  const float* sinks;
+  float* dterm;  // [T][H]
+  float* sterm;
+};
 
 // The spill (see SasBwdLayout): record 0 is all zeros, then record 1 + (t - t0) stride
 // + p for list position p of token t; a record is, per 32-head chunk, 64 B of
@@ -177,13 +159,14 @@ struct DqLds {
 // second barrier, the first tile was fetched after the query's rows, and the check for
 // infinities and NaNs took four instructions per value.  Measured, with the spill: 4 documents
 // of 608 .. 1,697 tokens, 128 heads, top-k 512, 1,390 -> 1,070 us; documents of 1,082
-// and 971 tokens, 64 heads, window only, d_qk 512, 232 -> 185 us.
+// and 971 tokens, 64 heads, window only, d_qk 512, 232 -> 185 us (and since it computes D
+// too 1,170 and 210 us).
 template <int DQK, int QT, bool SPILL>
 __device__ __forceinline__ void dq_unit(DqLds<DQK, SPILL>& sm, const int4 ur, int hg, const SasFwdArgs& a,
                                         const uint16_t* __restrict__ q, const uint16_t* __restrict__ dout,
                                         const uint64_t* __restrict__ addr_list,
                                         const int2* __restrict__ tok, const float* __restrict__ lse,
-                                        const float* __restrict__ dterm, const int* __restrict__ plan,
+                                        const SasBwdTerms& bt, const int* __restrict__ plan,
                                         float* __restrict__ dq, const SasBwdSpill& sp) {
   constexpr int DV = 512;
   constexpr bool ROPE = DQK > DV;
@@ -267,7 +250,7 @@ __device__ __forceinline__ void dq_unit(DqLds<DQK, SPILL>& sm, const int4 ur, in
   dma_rope(1, av1);
   asm volatile("" ::: "memory");
 
-  u32x4_t qf[KS], of[VKS];
+  u32x4_t qf[KS], of[VKS], ot[VKS];
   {
     const u32x4_t* qr = reinterpret_cast<const u32x4_t*>(q + th * DQK);
     const u32x4_t* orow = reinterpret_cast<const u32x4_t*>(dout + th * DV);
@@ -275,8 +258,12 @@ __device__ __forceinline__ void dq_unit(DqLds<DQK, SPILL>& sm, const int4 ur, in
     for (int ks = 0; ks < KS; ++ks) qf[ks] = qr[4 * ks + g];
 #pragma unroll
     for (int ks = 0; ks < VKS; ++ks) of[ks] = orow[4 * ks + g];
+    const u32x4_t* trow = reinterpret_cast<const u32x4_t*>(bt.out + th * DV);
+#pragma unroll
+    for (int ks = 0; ks < VKS; ++ks) ot[ks] = trow[4 * ks + g];
   }
-  const float lse2 = lse[th] * LOG2E, dh = dterm[th];
+  const float lse_h = lse[th], lse2 = lse_h * LOG2E, sink = bt.sinks[hc];
+  const float dl = bt.dlse ? bt.dlse[th] : 0.f;
   const float c = a.scale_log2;
   const float scale = c * 0.6931471805599453f;
   if constexpr (SPILL) {
@@ -295,6 +282,27 @@ __device__ __forceinline__ void dq_unit(DqLds<DQK, SPILL>& sm, const int4 ur, in
     if (__any(z != 0.f) && lane == 0) {
       sp.flags[1 + t] = 1;
       atomicAdd(sp.flags, 1);
+    }
+  }
+  // D: the diagonal of the 16 heads' dO out^T (fragments of a row are the same registers as
+  // an A and as a B operand): head h sits in lane (n = h, g = h >> 2), element h & 3
+  float dh;
+  {
+    bw_f32x4 d0 = bw_f32x4{0.f, 0.f, 0.f, 0.f}, d1 = d0;
+#pragma unroll
+    for (int ks = 0; ks < VKS; ks += 2) {
+      d0 = bw_mfma<QT>(of[ks], ot[ks], d0);
+      d1 = bw_mfma<QT>(of[ks + 1], ot[ks + 1], d1);
+    }
+    const int e = n16 & 3;
+    const float v0 = e & 1 ? d0[1] + d1[1] : d0[0] + d1[0], v1 = e & 1 ? d0[3] + d1[3] : d0[2] + d1[2];
+    // a gradient of the LSE: d lse / d s_j = P_j and d lse / d sink = P_sink, so it
+    // enters as dS = P (dP - (D - dlse)) and dsink = -P_sink (D - dlse)
+    dh = __shfl(e & 2 ? v1 : v0, n16 + 16 * (n16 >> 2)) - dl;
+    if (split == 0 && g == 0 && hvalid) {
+      bt.dterm[th] = dh;
+      // a sink of -inf has P_sink = 0 (lse may be -inf too when nothing is attended)
+      bt.sterm[th] = sink == -INFINITY || dh == 0.f ? 0.f : -__expf(sink - lse_h) * dh;
     }
   }
   // SPILL: the wave's P and dS go through LDS: lane (n16, g) writes its 8 keys of head
@@ -471,8 +479,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
                                                         const uint16_t* __restrict__ dout,
                                                         const uint64_t* __restrict__ addr_list,
                                                         const int2* __restrict__ tok,
-                                                        const float* __restrict__ lse,
-                                                        const float* __restrict__ dterm,
+                                                        const float* __restrict__ lse, SasBwdTerms bt,
                                                         const int* __restrict__ plan,
                                                         float* __restrict__ dq, SasBwdSpill sp) {
   __shared__ DqLds<DQK, SPILL> sm;
@@ -485,7 +492,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
   const bool ok = plan_matches(plan, a);
   asm volatile("" : "+s"(ur.x), "+s"(ur.y), "+s"(ur.z), "+s"(ur.w));
   if (!ok || u >= units) return;  // refused plan: prep zeroed dq
-  dq_unit<DQK, QT, SPILL>(sm, ur, hg, a, q, dout, addr_list, tok, lse, dterm, plan, dq, sp);
+  dq_unit<DQK, QT, SPILL>(sm, ur, hg, a, q, dout, addr_list, tok, lse, bt, plan, dq, sp);
 }
 
 // ---------------------------------------------------------------------------

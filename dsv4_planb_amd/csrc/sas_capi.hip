@@ -534,19 +534,18 @@ int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
   const int2* tok = w.tok;
   const uint64_t* addr = w.addr;
   int* flags = tiles ? reinterpret_cast<int*>(base + L.off_flags) : nullptr;
-  hipLaunchKernelGGL(f16 ? &sas::bwd_prep_kernel<1> : &sas::bwd_prep_kernel<0>,
-                     dim3(T * ((H + 3) / 4)), dim3(256), 0, s, a, p->head_dim_qk, plan, tok, go,
-                     static_cast<const uint16_t*>(t->out), t->lse, dlse, t->sinks, dterm, sterm, dq,
-                     flags);
+  hipLaunchKernelGGL(sas::bwd_prep_kernel, dim3(T * ((H + sas::BP_HEADS - 1) / sas::BP_HEADS)), dim3(256), 0, s,
+                     a, p->head_dim_qk, plan, tok, dterm, sterm, dq, flags);
   if ((rc = launch_status())) return rc;
   const dim3 grid(a.unit_cap * ((H + sas::BW_HEADS - 1) / sas::BW_HEADS));
   typedef void (*bwd_fn_t)(SasFwdArgs, const uint16_t*, const uint16_t*, const uint64_t*,
-                           const int2*, const float*, const float*, const int*, float*,
+                           const int2*, const float*, sas::SasBwdTerms, const int*, float*,
                            sas::SasBwdSpill);
   const bwd_fn_t fn = tiles ? (d576 ? (f16 ? &sas::bwd_dq_kernel<576, 1, true> : &sas::bwd_dq_kernel<576, 0, true>)
                                     : (f16 ? &sas::bwd_dq_kernel<512, 1, true> : &sas::bwd_dq_kernel<512, 0, true>))
                             : (d576 ? (f16 ? &sas::bwd_dq_kernel<576, 1, false> : &sas::bwd_dq_kernel<576, 0, false>)
                                     : (f16 ? &sas::bwd_dq_kernel<512, 1, false> : &sas::bwd_dq_kernel<512, 0, false>));
+  const sas::SasBwdTerms bt = {static_cast<const uint16_t*>(t->out), dlse, t->sinks, dterm, sterm};
   sas::SasBwdSpill sp = {};
   sas::SasTileArgs ta = {};
   if (tiles) {
@@ -573,7 +572,7 @@ int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
     sp.t0 = t0;
     sp.t1 = std::min(T, t0 + L.chunk_tokens);
     hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, a, q, go, addr, tok,
-                       static_cast<const float*>(t->lse), static_cast<const float*>(dterm), plan, dq, sp);
+                       static_cast<const float*>(t->lse), bt, plan, dq, sp);
     if ((rc = launch_status())) return rc;
     if (!tiles) break;
     hipLaunchKernelGGL(sas::bwd_items_kernel, dim3(1), dim3(1024), 0, s, a, ta, sp, plan);
