@@ -367,8 +367,9 @@ def measure(wl, steps, warmup, core_num=256, settle_s=0.25, sustain_s=0.0):
 
 # FLOPs per (row, head) of the backward.  Algorithmic (FlashAttention-2's
 # backward with P recomputed from the LSE): S = q K^T (2 d_qk), dP = dO V^T
-# (2 d_v), dq = dS K (2 d_qk), dK = dS^T q (2 d_qk), dV = P^T dO (2 d_v).  The
-# kernels run S and dP twice (once for dq, once for the pools' gradient).
+# (2 d_v), dq = dS K (2 d_qk), dK = dS^T q (2 d_qk), dV = P^T dO (2 d_v).  Without
+# key tiles (decode-like calls) the kernels run S and dP twice, once for dq and once for
+# the pools' gradient; with them the dq kernel hands P and dS on through the workspace.
 BWD_FLOP_DQ = 2 * D_QK + 2 * D_V + 2 * D_QK           # dq and dsinks
 BWD_FLOP_ALG = BWD_FLOP_DQ + 2 * D_QK + 2 * D_V       # dq, dsinks, dK, dV
 BWD_FLOP_EXEC = BWD_FLOP_DQ + 2 * D_QK + 2 * D_V + 2 * D_QK + 2 * D_V
@@ -391,12 +392,15 @@ def measure_backward(wl, steps, core_num=256, settle_s=0.25):
         res = {}
         for kv in (False, True):
             bufs = launch.backward_buffers(kv_grad=kv)
+            if not kv:
+                plain_ws = bufs["ws"].numel()
+            tiled = kv and bufs["ws"].numel() > plain_ws
             call = lambda: launch.backward_into(dout, None, bufs)  # noqa: E731
             _settle(call, settle_s, stream)
             us = _events_time(call, steps, stream)
             rows_heads = wl["rows_total"] * wl["H"]
             flop_alg = rows_heads * (BWD_FLOP_ALG if kv else BWD_FLOP_DQ)
-            flop_exec = rows_heads * (BWD_FLOP_EXEC if kv else BWD_FLOP_DQ)
+            flop_exec = rows_heads * (BWD_FLOP_DQ if not kv else BWD_FLOP_ALG if tiled else BWD_FLOP_EXEC)
             res["dq_dkv" if kv else "dq"] = dict(
                 call_us=round(us, 2), alg_flops=flop_alg, exec_flops=flop_exec,
                 tflops=round(flop_alg / (us * 1e-6) / 1e12, 2),
@@ -408,8 +412,9 @@ def measure_backward(wl, steps, core_num=256, settle_s=0.25):
             torch.cuda.empty_cache()
         res["dkv_us"] = round(res["dq_dkv"]["call_us"] - res["dq"]["call_us"], 2)
         # fp32 atomic adds of the pools' gradient per call: every (token, list row)
-        # adds one d_qk-wide row, summed over the heads first
-        res["dkv_atomic_bytes"] = int(wl["rows_total"] * D_QK * 4)
+        # adds one d_qk-wide row, summed over the heads first (with key tiles: one per
+        # tile and token group, whose number is the device's choice)
+        res["dkv_atomic_bytes"] = None if tiled else int(wl["rows_total"] * D_QK * 4)
     return res
 
 
