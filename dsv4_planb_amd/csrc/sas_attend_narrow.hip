@@ -620,8 +620,8 @@ __global__ __launch_bounds__(NW_NT, 1) void attend_narrow_kernel(
   sm.stamps = a.stamps;
   sm.t0 = __builtin_amdgcn_s_memrealtime();
   // The unit's record with the plan's header, before the header says whether the plan and
-  // the unit are sound (the grid is the call's own unit capacity, which the plan's buffer
-  // holds): one memory round trip for both, of the unit's three.
+  // the unit are sound: one memory round trip for both, of the unit's three.  (plan is the
+  // workspace's, which holds the grid's unit capacity; see resolve_kernel.)
   const int units = plan[PH_UNITS];
   const int* up = plan + SAS_PLAN_HDR + (size_t)SAS_TOK_W * a.T + (size_t)u * SAS_UNIT_W;
   int4 ur = make_int4(up[0], up[1], up[2], up[3]);

@@ -485,7 +485,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(SasFwdArgs a, const uint
   __shared__ DqLds<DQK, SPILL> sm;
   const int HG = (a.H + BW_HEADS - 1) / BW_HEADS;
   const int u = blockIdx.x / HG, hg = blockIdx.x - u * HG;
-  // (the unit's record with the plan's header: one memory round trip for both)
+  // (the unit's record with the plan's header: one memory round trip for both; plan is the
+  // workspace's, which holds the grid's unit capacity: see resolve_kernel)
   const int* up = plan + SAS_PLAN_HDR + (size_t)SAS_TOK_W * a.T + (size_t)u * SAS_UNIT_W;
   int4 ur = make_int4(up[0], up[1], up[2], up[3]);
   const int units = plan[PH_UNITS];

@@ -157,6 +157,8 @@ sas::SasResolveArgs resolve_args(const sas_params_t* p, const sas_tensors_t* t, 
   r.scale = w.scale;
   r.inv = nullptr;
   r.inv_rows = 0;
+  r.local = nullptr;
+  r.copies = 0;
   return r;
 }
 
@@ -217,6 +219,8 @@ int launch_attend(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
                   bool resolve, uint64_t* stamps = nullptr, bool cu_ends = false) {
   SasFwdArgs a = fwd_args(p, target);
   a.stamps = stamps;
+  // the two-wave kernel reads the workspace's plan (the resolver has copied a caller's to it)
+  if (narrow_heads(p, target)) plan = w.plan;
   sas::SasResolveArgs r = resolve_args(p, t, w, cu_ends);
   if (!resolve) r.addr = nullptr;
   r.rows = nullptr;  // the forward needs addresses only (sas_resolve also writes the codes)
@@ -236,9 +240,10 @@ int launch_attend(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
 
 // The resolver stage; codes: also write the row codes (the forward reads addresses
 // only; the backward and sas_debug_rows read the codes).  inv: also the inverse lists.
+// local: a caller's plan is copied to the workspace's, for kernels that read that one.
 int resolve_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
-                  size_t ws_bytes, sas_stream_t stream, bool codes, uint32_t* inv = nullptr,
-                  int inv_rows = 0, bool cu_ends = false) {
+                  size_t ws_bytes, sas_stream_t stream, bool codes, bool local,
+                  uint32_t* inv = nullptr, int inv_rows = 0, bool cu_ends = false) {
   int rc = sas_validate(p);
   if (rc) return rc;
   if ((rc = check_tensors(p, t))) return rc;
@@ -251,8 +256,14 @@ int resolve_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
   if (!codes) r.rows = nullptr;
   r.inv = inv;
   r.inv_rows = inv_rows;
-  hipLaunchKernelGGL(inv ? &sas::resolve_kernel<true> : &sas::resolve_kernel<false>, dim3(p->total_tokens), dim3(sas::RS_NT), 0,
-                     (hipStream_t)stream, fwd_args(p, target), plan, r);
+  if (local && plan != w.plan) {
+    const SasPlanLayout L = sas_plan_layout(p->total_tokens, target);
+    r.local = w.plan;
+    r.copies = (int)((L.off_split_tokens + sas::RS_COPY - 1) / sas::RS_COPY);
+  }
+  hipLaunchKernelGGL(inv ? &sas::resolve_kernel<true> : &sas::resolve_kernel<false>,
+                     dim3(p->total_tokens + r.copies), dim3(sas::RS_NT), 0, (hipStream_t)stream,
+                     fwd_args(p, target), plan, r);
   return launch_status();
 }
 
@@ -302,7 +313,9 @@ int forward_impl(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
   if (fused_resolution(p, target)) {
     if ((rc = launch_attend(p, t, plan, w, target, stream, nullptr, nullptr, true, nullptr, cu_ends))) return rc;
   } else {
-    if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, false, nullptr, 0, cu_ends))) return rc;
+    if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, false, narrow_heads(p, target), nullptr, 0,
+                            cu_ends)))
+      return rc;
     if ((rc = launch_attend(p, t, plan, w, target, stream, nullptr, nullptr, false, nullptr, cu_ends))) return rc;
   }
   return combine_stage(p, t, plan, ws, ws_bytes, stream, status_out);
@@ -424,7 +437,8 @@ int sas_plan(const sas_params_t* p, const int32_t* q_prefix, const int32_t* act_
 
 int sas_resolve(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
                 size_t ws_bytes, sas_stream_t stream) {
-  return resolve_stage(p, t, plan, ws, ws_bytes, stream, true);
+  if (!p) return SAS_ERR_NULL;
+  return resolve_stage(p, t, plan, ws, ws_bytes, stream, true, narrow_heads(p, target_units(p)));
 }
 
 int sas_attend_timed(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
@@ -526,7 +540,8 @@ int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
   const bool tiles = kv_grad && L.tile;
   const bool use_inv = tiles && p->scenario == 3 && L.cmp_rows > 0;
   uint32_t* inv = use_inv ? reinterpret_cast<uint32_t*>(base + L.off_inv) : nullptr;
-  if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, true, inv, L.cmp_rows))) return rc;
+  if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, true, true, inv, L.cmp_rows))) return rc;
+  plan = w.plan;  // (the resolver has copied a caller's to it)
   const SasFwdArgs a = fwd_args(p, target);
   const bool f16 = p->q_dtype == SAS_DT_FP16, d576 = p->head_dim_qk == 576;
   const uint16_t* q = static_cast<const uint16_t*>(t->q);

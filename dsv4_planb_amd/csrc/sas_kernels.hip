@@ -420,6 +420,8 @@ struct SasResolveArgs {
   // it is listed (high 16 bits; 0: not).  Entries below the token's threshold are set.
   uint32_t* inv;
   int inv_rows;
+  int* local;             // the workspace's plan, to which a caller's is copied (resolve_kernel)
+  int copies;             // by that many workgroups (0: no copy)
 };
 
 // List positions [lo, hi) of token t (its window rows, then its compressed rows)
@@ -654,15 +656,40 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
   return emitted;
 }
 
-// One workgroup (RS_NT threads) per token: its whole list.
+// The resolver, one workgroup (RS_NT threads) per token: its whole list.
+//
+// Ahead of those, with r.local, r.copies workgroups that copy the caller's plan (header,
+// token records, units) to the workspace's, which is as long as this call's plan whatever
+// the caller's buffer holds: the entry points take no plan size, and a plan built for fewer
+// tokens or a smaller target is a shorter buffer, so nothing past its header is read unless
+// the header matches (a refused plan leaves a header of zeros).  The kernels behind the
+// resolver then read a unit's record together with the header that vouches for it, one
+// memory round trip of each unit's start: a window-only prefill of 8,192 tokens (64
+// heads, d_qk 512, fp16) took 1 to 2% longer where they read a caller's header first (332
+// -> 336 .. 339 us).  (In workgroups of their own: at the end of every token's the copy
+// made the resolver 2 us longer.)
+constexpr int RS_COPY = 8 * RS_NT;  // plan entries per copying workgroup
 template <bool INV>
 __global__ __launch_bounds__(RS_NT) void resolve_kernel(SasFwdArgs a, const int* __restrict__ plan,
                                                         SasResolveArgs r) {
   __shared__ RsShared<RS_NT> sh;
-  const int t = blockIdx.x;
   // A plan built for other arguments is refused: every token resolves to no rows,
   // the attention kernel writes zeros and the combine kernel sets the status word.
   const bool plan_ok = plan_matches(plan, a);
+  const int t = (int)blockIdx.x - r.copies;
+  if (t < 0) {
+    const int64_t n = SAS_PLAN_HDR + (int64_t)a.T * SAS_TOK_W +
+                      (int64_t)min(plan[PH_UNITS], a.unit_cap) * SAS_UNIT_W;
+    const int64_t i0 = (int64_t)blockIdx.x * RS_COPY + threadIdx.x;
+    if (!plan_ok) {
+      if (i0 < SAS_PLAN_HDR) r.local[i0] = 0;
+      return;
+    }
+#pragma unroll
+    for (int k = 0; k < RS_COPY / RS_NT; ++k)
+      if (i0 + k * RS_NT < n) r.local[i0 + k * RS_NT] = plan[i0 + k * RS_NT];
+    return;
+  }
   const int* tk = plan + SAS_PLAN_HDR + (size_t)t * SAS_TOK_W;
   int nwin = 0;
   const int n = resolve_rows<INV, RS_NT>(a, tk, plan_ok, t, 0, a.list_stride, sh, r, nwin);
@@ -935,9 +962,10 @@ __global__ __launch_bounds__(64 * COMBINE_WAVES, COMBINE_WGS_PER_CU<QT>) void co
       if (status_out) *status_out = st;
     }
   }
-  // The split token's record (token, split count, first slot) is loaded with the
-  // plan header, before the header says how many split tokens there are: its
-  // index is clamped into the list, and a record past the count is never used.
+  if (!plan_ok) return;  // refused plan: the attention kernel wrote zeros (see plan_unit)
+  // The split token's record (token, split count, first slot) is loaded before it is
+  // known whether there are that many split tokens: its index is clamped into the
+  // list, and a record past the count is never used.
   auto split_record = [&](int i) {
     const int ic = min(i, (int)L.split_cap - 1);
     return make_int3(plan[L.off_split_tokens + ic], plan[L.off_split_meta + 2 * ic],
@@ -948,7 +976,6 @@ __global__ __launch_bounds__(64 * COMBINE_WAVES, COMBINE_WGS_PER_CU<QT>) void co
   // while this one merges: one memory round trip per item.
   const int stride = gridDim.x * COMBINE_WAVES;
   int3 rec = split_record(wave / H);
-  if (!plan_ok) return;  // refused plan: the attention kernel wrote zeros
   const int items = plan[PH_NSPLIT_TOKENS] * H;  // (split token, head) pairs
   const int lane = threadIdx.x & 63;
   for (int item = wave; item < items; item += stride) {

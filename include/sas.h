@@ -146,7 +146,8 @@ int sas_plan(const sas_params_t* p, const int32_t* q_prefix, const int32_t* act_
  * as zeros), and every token the call's q_prefix / act_q give to another batch or
  * position (that token's outputs written as zeros); the first int32 of the
  * workspace, the status word written by every call, then reads SAS_ERR_PLAN
- * instead of SAS_OK. */
+ * instead of SAS_OK.  A plan buffer shorter than this call's (built for fewer tokens or
+ * a smaller target) is refused the same way: nothing past its header is read. */
 int sas_forward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan,
                 void* workspace, size_t workspace_bytes, sas_stream_t stream);
 /* sas_forward with t->act_q_lens holding each sequence's cumulative end (the
@@ -155,7 +156,7 @@ int sas_forward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* pl
  * nothing to form the lengths. */
 int sas_forward_cu(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan,
                    void* workspace, size_t workspace_bytes, sas_stream_t stream);
-/* The stages of sas_forward, for timing and debugging (same workspace).
+/* The stages of sas_forward, for timing and debugging (same workspace, same plan).
  * sas_resolve writes every token's row lists (codes too) and counts; sas_attend
  * launches the attention dispatch exactly as sas_forward does (where the forward
  * lets the units resolve their own rows, so does sas_attend) and writes the output
