@@ -241,8 +241,10 @@ class SasLaunch:
         g = dout.to(device=dev, dtype=q_dt).reshape(T, H, p.head_dim_v).contiguous()
         gl = None if dlse is None else dlse.to(device=dev, dtype=torch.float32).reshape(T, H).contiguous()
         bufs = self.backward_buffers(kv_grad)
+        # The workspace (the spill: up to 2 GiB and more) and the converted gradients go back to
+        # the allocator here, which hands them on in stream order; kept on the launch, every
+        # layer of a model would hold its own until its graph is released.
         self.backward_into(g, gl, bufs)
-        self._bwd_keep = (g, gl, bufs["ws"])  # alive until the stream has used them
         if kv_grad:
             return bufs["dq"], bufs["dsinks"], bufs["d_ori"], bufs["d_cmp"]
         return bufs["dq"], bufs["dsinks"]

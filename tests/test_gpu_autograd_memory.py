@@ -39,23 +39,23 @@ def test_a_layers_backward_workspace_is_given_back(layers):
     cmp_ = d["cmp_kv"].detach().requires_grad_()
     qs = [d["q"].detach().clone().requires_grad_() for _ in range(layers)]
     outs = [_call(c, d, q, ori, cmp_) for q in qs]
-    loss = sum(o.float().square().sum() for o in outs)
+    g = torch.randn(outs[0].shape, device="cuda", generator=torch.Generator("cuda").manual_seed(6)).to(outs[0].dtype)
     # one layer's workspace, from a launch of the same call
     need = _workspace(c, d)
     assert need > 64 << 20
     gc.collect()
     torch.cuda.synchronize()
     before = torch.cuda.memory_allocated()
-    loss.backward()
+    torch.autograd.backward(outs, [g] * layers)
     torch.cuda.synchronize()
     grads = sum(x.grad.numel() * x.grad.element_size() for x in [*qs, ori, cmp_])
     held = torch.cuda.memory_allocated() - before - grads
     print(f"held beside the gradients: {held / 2**20:.1f} MiB; a workspace: {need / 2**20:.1f} MiB", flush=True)
-    assert held < need // 2  # (the loss, and with it every layer's node, is alive)
+    assert held < need // 16  # (the outputs, and with them every layer's node, are alive)
     # the released workspaces were not reused too early: every layer has the same gradient
     for q in qs[1:]:
         assert torch.equal(q.grad, qs[0].grad)
-    del loss, outs
+    del outs
 
 
 def _workspace(c, d):
