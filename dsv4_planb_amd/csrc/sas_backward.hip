@@ -80,16 +80,16 @@ __device__ __forceinline__ float dot2_zero(uint32_t v, uint32_t zero, float acc)
   }
 }
 
-// What the dq kernel leaves out, per (token, BP_HEADS heads): the terms of tokens that no
+// What the dq kernel leaves out, per (token from t0 on, BP_HEADS heads): the terms of tokens that no
 // batch owns (or whose plan is refused), and the zeros of their dq rows and of those that
 // several units add to; and the flags of a call whose P and dS are spilled (else null).
 constexpr int BP_HEADS = 64;
-__global__ __launch_bounds__(256) void bwd_prep_kernel(SasFwdArgs a, int dqk, const int* __restrict__ plan,
+__global__ __launch_bounds__(256) void bwd_prep_kernel(SasFwdArgs a, int dqk, int t0, const int* __restrict__ plan,
                                                        const int2* __restrict__ tok,
                                                        float* __restrict__ dterm, float* __restrict__ sterm,
                                                        float* __restrict__ dq, int* __restrict__ flags) {
   const int HB = (a.H + BP_HEADS - 1) / BP_HEADS;
-  const int t = blockIdx.x / HB, h0 = (blockIdx.x - t * HB) * BP_HEADS;
+  const int tb = blockIdx.x / HB, t = t0 + tb, h0 = (blockIdx.x - tb * HB) * BP_HEADS;
   const int tid = threadIdx.x, nh = min(BP_HEADS, a.H - h0);
   if (flags && tid == 0 && h0 == 0) {
     flags[1 + t] = 0;

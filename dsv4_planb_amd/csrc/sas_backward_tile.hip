@@ -46,7 +46,7 @@ struct SasTileArgs {
   const int* seqused_kv;
   const int* ori_bt;
   const int* cmp_bt;
-  const uint32_t* inv;  // scenario 3: the resolver's inverse lists, [T][cmp_rows]
+  const uint32_t* inv;  // scenario 3: the resolver's inverse lists, [the run's tokens][cmp_rows]
   int cmp_rows;         // compressed rows covered by tiles (0: none)
   int item_cap;
   int workers;          // workgroups of bwd_dkv_tile_kernel
@@ -245,7 +245,7 @@ __device__ __forceinline__ void dkv_tile(TileLds<DQK>& sm, const int4 it, const 
       const int hi = __builtin_amdgcn_readlane(v_hi, i), c = __builtin_amdgcn_readlane(v_cnt, i);
       int m = 0;
       if (c) {
-        const uint32_t* iv = ta.inv + (size_t)(first + i) * ta.cmp_rows;
+        const uint32_t* iv = ta.inv + (size_t)(first + i - sp.t0) * ta.cmp_rows;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
           const int p = p0 + 64 * k + lane;
@@ -316,7 +316,7 @@ __device__ __forceinline__ void dkv_tile(TileLds<DQK>& sm, const int4 it, const 
   // the paths join.
   auto load_inv = [&](int i) -> uint32_t {
     typedef __attribute__((address_space(1))) const uint8_t g_u8;
-    const g_u8* iv = use_inv ? (const g_u8*)(uintptr_t)(ta.inv + (size_t)(first + i) * ta.cmp_rows)
+    const g_u8* iv = use_inv ? (const g_u8*)(uintptr_t)(ta.inv + (size_t)(first + i - sp.t0) * ta.cmp_rows)
                              : (const g_u8*)(uintptr_t)sp.data;
     // (positions past the token's last read that one: set_rows drops them)
     const int hi = use_inv ? __builtin_amdgcn_readlane(v_hi, i) : 0;

@@ -155,6 +155,7 @@ sas::SasResolveArgs resolve_args(const sas_params_t* p, const sas_tensors_t* t, 
   r.ori_scale = t->ori_kv_scale;
   r.cmp_scale = t->cmp_kv_scale;
   r.scale = w.scale;
+  r.t0 = 0;
   r.inv = nullptr;
   r.inv_rows = 0;
   r.local = nullptr;
@@ -241,9 +242,11 @@ int launch_attend(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
 // The resolver stage; codes: also write the row codes (the forward reads addresses
 // only; the backward and sas_debug_rows read the codes).  inv: also the inverse lists.
 // local: a caller's plan is copied to the workspace's, for kernels that read that one.
+// t0, t1: the tokens (t1 < 0: all).
 int resolve_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* plan, void* ws,
                   size_t ws_bytes, sas_stream_t stream, bool codes, bool local,
-                  uint32_t* inv = nullptr, int inv_rows = 0, bool cu_ends = false) {
+                  uint32_t* inv = nullptr, int inv_rows = 0, bool cu_ends = false, int t0 = 0,
+                  int t1 = -1) {
   int rc = sas_validate(p);
   if (rc) return rc;
   if ((rc = check_tensors(p, t))) return rc;
@@ -256,13 +259,15 @@ int resolve_stage(const sas_params_t* p, const sas_tensors_t* t, const int32_t* 
   if (!codes) r.rows = nullptr;
   r.inv = inv;
   r.inv_rows = inv_rows;
+  r.t0 = t0;
+  if (t1 < 0) t1 = p->total_tokens;
   if (local && plan != w.plan) {
     const SasPlanLayout L = sas_plan_layout(p->total_tokens, target);
     r.local = w.plan;
     r.copies = (int)((L.off_split_tokens + sas::RS_COPY - 1) / sas::RS_COPY);
   }
   hipLaunchKernelGGL(inv ? &sas::resolve_kernel<true> : &sas::resolve_kernel<false>,
-                     dim3(p->total_tokens + r.copies), dim3(sas::RS_NT), 0, (hipStream_t)stream,
+                     dim3(t1 - t0 + r.copies), dim3(sas::RS_NT), 0, (hipStream_t)stream,
                      fwd_args(p, target), plan, r);
   return launch_status();
 }
@@ -540,8 +545,6 @@ int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
   const bool tiles = kv_grad && L.tile;
   const bool use_inv = tiles && p->scenario == 3 && L.cmp_rows > 0;
   uint32_t* inv = use_inv ? reinterpret_cast<uint32_t*>(base + L.off_inv) : nullptr;
-  if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, true, true, inv, L.cmp_rows))) return rc;
-  plan = w.plan;  // (the resolver has copied a caller's to it)
   const SasFwdArgs a = fwd_args(p, target);
   const bool f16 = p->q_dtype == SAS_DT_FP16, d576 = p->head_dim_qk == 576;
   const uint16_t* q = static_cast<const uint16_t*>(t->q);
@@ -549,9 +552,6 @@ int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
   const int2* tok = w.tok;
   const uint64_t* addr = w.addr;
   int* flags = tiles ? reinterpret_cast<int*>(base + L.off_flags) : nullptr;
-  hipLaunchKernelGGL(sas::bwd_prep_kernel, dim3(T * ((H + sas::BP_HEADS - 1) / sas::BP_HEADS)), dim3(256), 0, s,
-                     a, p->head_dim_qk, plan, tok, dterm, sterm, dq, flags);
-  if ((rc = launch_status())) return rc;
   const dim3 grid(a.unit_cap * ((H + sas::BW_HEADS - 1) / sas::BW_HEADS));
   typedef void (*bwd_fn_t)(SasFwdArgs, const uint16_t*, const uint16_t*, const uint64_t*,
                            const int2*, const float*, sas::SasBwdTerms, const int*, float*,
@@ -582,10 +582,19 @@ int sas_backward(const sas_params_t* p, const sas_tensors_t* t, const int32_t* p
     ta.want_cmp = L.cmp_rows > 0 && d_cmp_kv != nullptr;
     ta.items = reinterpret_cast<int4*>(base + L.off_items);
   }
-  // the tokens in runs that the spill holds (one run where nothing is spilled)
-  for (int t0 = 0; t0 < T; t0 += L.chunk_tokens) {
+  // the tokens in runs that the spill and the inverse lists hold (one run where nothing is
+  // spilled)
+  const int chunk = tiles ? L.chunk_tokens : T;
+  for (int t0 = 0; t0 < T; t0 += chunk) {
     sp.t0 = t0;
-    sp.t1 = std::min(T, t0 + L.chunk_tokens);
+    sp.t1 = std::min(T, t0 + chunk);
+    if ((rc = resolve_stage(p, t, plan, ws, ws_bytes, stream, true, t0 == 0, inv, L.cmp_rows, false, t0, sp.t1)))
+      return rc;
+    plan = w.plan;  // (the first run's resolver has copied a caller's to it)
+    const int run = sp.t1 - t0;
+    hipLaunchKernelGGL(sas::bwd_prep_kernel, dim3(run * ((H + sas::BP_HEADS - 1) / sas::BP_HEADS)), dim3(256), 0, s,
+                       a, p->head_dim_qk, t0, plan, tok, dterm, sterm, dq, flags);
+    if ((rc = launch_status())) return rc;
     hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, a, q, go, addr, tok,
                        static_cast<const float*>(t->lse), bt, plan, dq, sp);
     if ((rc = launch_status())) return rc;

@@ -135,10 +135,10 @@ SAS_HD static inline SasWsLayout sas_ws_layout(int64_t T, int64_t K, int64_t H, 
 // ---- backward workspace: the forward's, then (bytes, each region 256-B aligned) ----
 // The KV pools' gradient by key tiles (bwd_dkv_tile_kernel) reads every row's P and dS
 // back from memory: the dq kernel spills them, one record per list position (2 B dS and
-// 2 B P per head, heads padded to whole 32-head chunks).  The spill is bounded: the
-// tokens are taken in runs of chunk_tokens.
+// 2 B P per head, heads padded to whole 32-head chunks), and in scenario 3 the resolver's
+// inverse lists.  Both are bounded together: the tokens are taken in runs of chunk_tokens.
 #define SAS_BWD_KEYS 128                          // keys per tile item
-#define SAS_BWD_SPILL_BYTES ((size_t)2 << 30)     // spill bound (at least one token)
+#define SAS_BWD_SPILL_BYTES ((size_t)2 << 30)     // bound of a run's spill and inverse lists
 #define SAS_BWD_MIN_GROUP 8                       // fewest tokens per tile item
 #define SAS_BWD_MAX_B 2048                        // sequences the item list handles
 // Tiles for compressed rows when the table holds at most this times K rows: a tile visit
@@ -179,7 +179,8 @@ SAS_HD static inline SasBwdLayout sas_bwd_layout(size_t fwd_total, int64_t T, in
     L.cmp_rows = (int)cmp_cap;
     stride = full;
   }
-  const size_t per_token = (size_t)stride * (size_t)L.row_bytes;
+  const size_t inv_bytes = scenario == 3 ? (size_t)L.cmp_rows * 4 : 0;  // per token
+  const size_t per_token = (size_t)stride * (size_t)L.row_bytes + inv_bytes;
   if (per_token > SAS_BWD_SPILL_BYTES) L.tile = L.cmp_rows = 0;
   L.stride = (int)stride;
   L.off_flags = L.off_inv = L.off_items = L.off_spill = L.total = L.base_total;
@@ -203,7 +204,7 @@ SAS_HD static inline SasBwdLayout sas_bwd_layout(size_t fwd_total, int64_t T, in
   L.off_flags = L.total;
   L.total += sas_align256((size_t)(T + 1) * 4);
   L.off_inv = L.total;
-  if (scenario == 3) L.total += sas_align256((size_t)T * (size_t)L.cmp_rows * 4);
+  L.total += sas_align256((size_t)chunk * inv_bytes);
   L.off_items = L.total;
   L.total += sas_align256((size_t)(L.item_cap + 1) * 16);
   L.off_spill = L.total;

@@ -415,9 +415,10 @@ struct SasResolveArgs {
   const float* ori_scale;
   const float* cmp_scale;
   float* scale;           // fp8: s, then (T * list_stride on) 1 / s; nullptr for 16-bit KV
-  // INV: scenario 3's inverse list, [T][inv_rows]: for compressed row j of the token's
-  // sequence, the list position of its first occurrence (low 16 bits) and how often
-  // it is listed (high 16 bits; 0: not).  Entries below the token's threshold are set.
+  int t0;                 // the launch's first token
+  // INV: scenario 3's inverse list, [tokens of the launch][inv_rows]: for compressed row j of
+  // the token's sequence, the list position of its first occurrence (low 16 bits) and how
+  // often it is listed (high 16 bits; 0: not).  Entries below the token's threshold are set.
   uint32_t* inv;
   int inv_rows;
   int* local;             // the workspace's plan, to which a caller's is copied (resolve_kernel)
@@ -547,7 +548,7 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
   g_u32* inv = nullptr;
   if constexpr (INV) {
     if (r.inv) {
-      inv = (g_u32*)(uintptr_t)(r.inv + (size_t)t * r.inv_rows);
+      inv = (g_u32*)(uintptr_t)(r.inv + (size_t)(t - r.t0) * r.inv_rows);
       for (int i = tid; i < min(thr, r.inv_rows); i += NT) inv[i] = 0;
       __syncthreads();  // the zeros are in place before the first count below
     }
@@ -676,8 +677,8 @@ __global__ __launch_bounds__(RS_NT) void resolve_kernel(SasFwdArgs a, const int*
   // A plan built for other arguments is refused: every token resolves to no rows,
   // the attention kernel writes zeros and the combine kernel sets the status word.
   const bool plan_ok = plan_matches(plan, a);
-  const int t = (int)blockIdx.x - r.copies;
-  if (t < 0) {
+  const int t = (int)blockIdx.x - r.copies + r.t0;
+  if ((int)blockIdx.x < r.copies) {
     const int64_t n = SAS_PLAN_HDR + (int64_t)a.T * SAS_TOK_W +
                       (int64_t)min(plan[PH_UNITS], a.unit_cap) * SAS_UNIT_W;
     const int64_t i0 = (int64_t)blockIdx.x * RS_COPY + threadIdx.x;

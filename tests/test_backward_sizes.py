@@ -9,7 +9,7 @@ import pytest
 from dsv4_planb_amd import _lib
 from tests.test_capi import _good
 
-BOUND = 2 << 30  # bytes of spilled P and dS per run of tokens
+BOUND = 2 << 30  # bytes of spilled P and dS and of inverse lists per run of tokens
 
 
 def _size(p, kv_grad):
@@ -34,10 +34,23 @@ def test_the_spill_keeps_to_its_bound(T, B, H, topk):
         return
     cmp_rows = 64 * 128 if 64 * 128 <= 6 * topk else 0
     rows = topk if cmp_rows else 0
-    per_token = (128 + rows + 31) // 32 * 32 * ((H + 31) // 32 * 128)
-    # beside the spill: a flag per token, the inverse lists, the items (at most one per 8
-    # tokens and sequence and per tile) and each region's alignment
+    per_token = (128 + rows + 31) // 32 * 32 * ((H + 31) // 32 * 128) + 4 * cmp_rows
+    # beside them: a flag per token, the items (at most one per 8 tokens and sequence and per
+    # tile) and each region's alignment
     tiles = (127 + 64) // 128 + 2 + (cmp_rows + 127) // 128
-    beside = 4 * (T + 1) + 4 * T * cmp_rows + 16 * ((T // 8 + B + 1) * tiles + 1) + 4 * 256
+    beside = 4 * (T + 1) + 16 * ((T // 8 + B + 1) * tiles + 1) + 4 * 256
     assert extra <= min(BOUND, T * per_token) + per_token // 100 + 1024 + beside
     assert extra >= min(BOUND // 2, T * per_token) - per_token
+
+
+# tables of 6 K compressed rows (the most that tiles take): inverse lists of every token would
+# be 3 to 9 GiB
+@pytest.mark.parametrize("T,B,H", [(65536, 1, 128), (131072, 4, 128), (200000, 1, 16)])
+def test_long_calls_keep_to_the_bound(T, B, H):
+    p = _good(total_tokens=T, batch=B, num_heads_q=H, topk=2048, cmp_table_len=96, cmp_block_size=128,
+              cmp_block_stride=128 * 576)
+    extra = _size(p, 1) - _size(p, 0)
+    assert extra > BOUND // 2  # (tiles for the compressed rows)
+    # the flags, and at most an item per 8 tokens of a run and per tile (12288 / 128 + 3)
+    run = BOUND // (2176 * ((H + 31) // 32 * 128) + 4 * 12288)
+    assert extra <= BOUND + 4 * (T + 1) + 16 * ((run // 8 + B + 1) * 99 + 1) + 8 * 256

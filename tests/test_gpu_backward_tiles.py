@@ -62,6 +62,18 @@ def test_tiles_match_f64_gradient(name, build):
     _check_pools(f"tiles_{name}", c, d_ori, d_cmp, dori_ex, dcmp_ex)
 
 
+def test_the_queries_gradient_alone_takes_every_run():
+    """dq and dsinks without the pools' gradient, of a call whose spill would take two runs."""
+    c = make_case(B=1, H=16, seq_kv=[1090], q_per_seq=[1090], scenario=3, K=16384, seed=206)
+    launch, _, _ = _launch(c)
+    g, _ = _dout(c, seed=9)
+    with_pools = launch.backward(g.cuda(), kv_grad=True)
+    alone = launch.backward(g.cuda())
+    torch.cuda.synchronize()
+    # (no token is split: no atomics in dq)
+    assert torch.equal(alone[0], with_pools[0]) and torch.equal(alone[1], with_pools[1])
+
+
 def test_an_infinite_gradient_stays_with_the_rows_its_token_reads():
     """One element of one token's dO is infinite: the rows that token attends may be
     anything, every other row is the gradient without that token."""
