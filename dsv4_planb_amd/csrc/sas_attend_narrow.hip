@@ -256,7 +256,8 @@ __device__ __forceinline__ bool narrow_unit(
             [l4] "s"((uint32_t)ra[4]), [h4] "s"((uint32_t)(ra[4] >> 32)),
             [l5] "s"((uint32_t)ra[5]), [h5] "s"((uint32_t)(ra[5] >> 32)),
             [l6] "s"((uint32_t)ra[6]), [h6] "s"((uint32_t)(ra[6] >> 32)),
-            [l7] "s"((uint32_t)ra[7]), [h7] "s"((uint32_t)(ra[7] >> 32)));
+            [l7] "s"((uint32_t)ra[7]), [h7] "s"((uint32_t)(ra[7] >> 32))
+          : "scc");  // (the shifts of exec)
       const uint64_t src = (((uint64_t)hi << 32) | lo) + vrope;
       const uint32_t m0 = (uint32_t)(uintptr_t)dst;
       uint32_t keep;  // the compiler's own value of m0

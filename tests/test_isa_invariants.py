@@ -123,3 +123,27 @@ def test_narrow_tile_loop_keeps_dmas_in_flight(asm):
         assert not waits, (name[:60], waits[:3])
         checked += 1
     assert checked == 4
+
+
+# scalar instructions that write SCC (moves, selects, multiplies, loads, waits and branches
+# do not)
+_WRITES_SCC = re.compile(r"\bs_(add|addc|sub|subb|absdiff|abs|min|max|and|or|xor|not|nand|nor|xnor|andn[12]|orn[12]|"
+                         r"lsh[lr]\d?|ashr|bfe|bcnt\d|wqm|quadmask|cmp|cmpk|bitcmp\d|addk)_")
+
+
+def test_assembly_that_writes_scc_says_so():
+    """An asm statement whose instructions write SCC names it in its clobbers: otherwise the
+    compiler may keep a comparison's result in SCC across the statement."""
+    checked = 0
+    for f in sorted(os.listdir(B.CSRC)):
+        text = open(os.path.join(B.CSRC, f)).read() if f.endswith((".hip", ".h")) else ""
+        for m in re.finditer(r"\basm\s+volatile\s*\(", text):
+            depth, i = 1, m.end()
+            while depth:
+                depth += {"(": 1, ")": -1}.get(text[i], 0)
+                i += 1
+            stmt = text[m.start():i]
+            checked += 1
+            if _WRITES_SCC.search(stmt):
+                assert '"scc"' in stmt, (f, text[:m.start()].count("\n") + 1)
+    assert checked > 50
