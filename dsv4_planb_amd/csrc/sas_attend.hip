@@ -1238,7 +1238,7 @@ __global__ __launch_bounds__(256, 1) void attend_kernel(
     float* __restrict__ lse, float* __restrict__ ws_o, float* __restrict__ ws_ml,
     SasResolveArgs rs) {
   __shared__ __attribute__((aligned(16))) AttendLds<DQK, KV8> sm;
-  static_assert(sizeof(RsShared<256>) <= sizeof(sm.tiles), "the resolution borrows the tile ring");
+  static_assert(sizeof(RsShared) <= sizeof(sm.tiles), "the resolution borrows the tile ring");
   const int u = blockIdx.x;
   // (every thread writes the same value, so each one's read at the end sees it,
   // whatever barriers the unit's path has)
@@ -1273,8 +1273,8 @@ __global__ __launch_bounds__(256, 1) void attend_kernel(
     const bool last = split < 0 || split == tk[TK_SPLITS] - 1;
     own_hi = last ? a.list_stride : min(ur[2], a.list_stride);
     int nwin = 0;
-    const int nc = resolve_rows<false, 256>(a, tk, true, t, ur[1], own_hi,
-                                *reinterpret_cast<RsShared<256>*>(sm.tiles), rs, nwin);
+    const int nc = resolve_rows<false>(a, tk, true, t, ur[1], own_hi,
+                                       *reinterpret_cast<RsShared*>(sm.tiles), rs, nwin);
     live = make_int2(nwin, nwin < 0 ? 0 : nc);
     if (rs.tok && threadIdx.x == 0 && last) rs.tok[t] = live;
     // Every wave's stores have reached L2 before any wave reads the lists back

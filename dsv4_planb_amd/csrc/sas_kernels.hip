@@ -374,9 +374,10 @@ __device__ __forceinline__ int paged_code(const int* __restrict__ bt_row, int ta
   return (page < 0 || page >= block_num) ? -1 : page * block_size + (pos - blk * block_size);
 }
 
-// A token is resolved by one workgroup of NT threads: the resolver's own (RS_NT), or
-// the attention workgroup of one of its units (128 or 256).
+// A token is resolved by one workgroup of RS_NT threads: the resolver's own, or the
+// four-wave attention kernel's of one of its units.
 constexpr int RS_NT = 256;
+constexpr int RS_WAVES = RS_NT / 64;
 
 // Workgroup barrier for the resolver: its threads exchange data only through LDS,
 // so it waits for LDS operations alone.  (__syncthreads() would also drain every
@@ -384,16 +385,15 @@ constexpr int RS_NT = 256;
 __device__ __forceinline__ void rs_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
-constexpr int RS_PASS = 2048;  // index slots per pass: RS_PASS / NT slabs of NT
+constexpr int RS_PER = 8;  // slabs of RS_NT index slots per pass
 
 constexpr int RS_CBT_LDS = 4096;  // compressed block-table entries staged in LDS
 
 // LDS of one token's resolution (the attention kernel lends it the start of its
 // tile ring, which is empty until the unit's first DMA).
-template <int NT>
 struct RsShared {
-  int wmin[NT / 64];
-  int cnt[RS_PASS / NT][NT / 64];
+  int wmin[RS_WAVES];
+  int cnt[RS_PER][RS_WAVES];
   int cbt[RS_CBT_LDS];
 };
 
@@ -426,9 +426,9 @@ struct SasResolveArgs {
 };
 
 // List positions [lo, hi) of token t (its window rows, then its compressed rows)
-// resolved into codes, pool addresses and (fp8) scales, by the workgroup's NT
+// resolved into codes, pool addresses and (fp8) scales, by the workgroup's RS_NT
 // threads.  The first min(K, thr) index slots are taken in passes of RS_PER slabs
-// of NT slots; thread i owns slot i of every slab, so each load and store
+// of RS_NT slots; thread i owns slot i of every slab, so each load and store
 // instruction of a wave covers 64 consecutive slots.  The first -1 (a block-wide
 // minimum) ends the list, ids outside [0, thr) are skipped, and the survivors keep
 // their slot order: a wave ranks its survivors of a slab with one ballot, and the
@@ -443,10 +443,9 @@ struct SasResolveArgs {
 // reuses its metadata).  Where the call's q_prefix / act_q no longer give the token
 // to batch b at position s (or give a token the plan left unowned to its candidate
 // batch), the token is refused: nwin_live = -1, nothing is resolved.
-template <bool INV, int NT>
+template <bool INV>
 __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, int t, int lo, int hi,
-                            RsShared<NT>& sh, const SasResolveArgs& r, int& nwin_live) {
-  constexpr int RS_PER = RS_PASS / NT, RS_WAVES = NT / 64;
+                            RsShared& sh, const SasResolveArgs& r, int& nwin_live) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, w = tid >> 6;
   const int* ir = r.idx + (size_t)t * a.K;
@@ -455,7 +454,7 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
   auto load_slots = [&](int (&v)[RS_PER], int c0, int bound) {
 #pragma unroll
     for (int k = 0; k < RS_PER; ++k) {
-      const int sl = c0 + k * NT + tid;
+      const int sl = c0 + k * RS_NT + tid;
       v[k] = sl < bound ? ir[sl] : -2;
     }
   };
@@ -494,10 +493,10 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
   const int* cbt_g = r.cmp_bt + (size_t)b * a.cmp_table_len;
   const bool cbt_lds = a.scenario >= 2 && a.cmp_table_len <= RS_CBT_LDS;
   if (cbt_lds)
-    for (int i = tid; i < a.cmp_table_len; i += NT) sh.cbt[i] = cbt_g[i];
+    for (int i = tid; i < a.cmp_table_len; i += RS_NT) sh.cbt[i] = cbt_g[i];
   const int* obt = r.ori_bt + (size_t)b * a.ori_table_len;
   auto window = [&](int nwin, int winlo) {
-    for (int p = lo + tid; p < min(hi, nwin); p += NT) {
+    for (int p = lo + tid; p < min(hi, nwin); p += RS_NT) {
       const int code = paged_code(obt, a.ori_table_len, a.ori_block_size, a.ori_block_num, winlo + p);
       if (out) out[p] = code;
       aout[p] = code_addr(code, r.ori_kv, a.ori_block_size, a.ori_block_stride, a.ori_row_stride, r.esz);
@@ -530,7 +529,7 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
     // One loop per source of the table row: a pointer that may be either (LDS or
     // global) turns its loads into FLAT instructions.
     auto cmp_rows = [&](const int* bt) {
-      for (int j = jlo + tid; j < min(n, jhi); j += NT) {
+      for (int j = jlo + tid; j < min(n, jhi); j += RS_NT) {
         const int code = paged_code(bt, a.cmp_table_len, a.cmp_block_size, a.cmp_block_num, j);
         if (out) out[nwin + j] = code;
         aout[nwin + j] = code_addr(code, r.cmp_kv, a.cmp_block_size, a.cmp_block_stride, a.cmp_row_stride, r.esz);
@@ -549,19 +548,19 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
   if constexpr (INV) {
     if (r.inv) {
       inv = (g_u32*)(uintptr_t)(r.inv + (size_t)(t - r.t0) * r.inv_rows);
-      for (int i = tid; i < min(thr, r.inv_rows); i += NT) inv[i] = 0;
+      for (int i = tid; i < min(thr, r.inv_rows); i += RS_NT) inv[i] = 0;
       __syncthreads();  // the zeros are in place before the first count below
     }
   }
-  // Passes of RS_PER slabs of NT slots; the terminator, the survivors and their
+  // Passes of RS_PER slabs of RS_NT slots; the terminator, the survivors and their
   // slot-order positions come from ballots and two LDS exchanges per pass.
   int emitted = 0;  // compressed rows found so far (block-uniform)
   const uint64_t below = (1ull << lane) - 1;  // lanes ranked before this one
-  for (int c0 = 0; c0 < limit && emitted < jhi; c0 += NT * RS_PER) {
+  for (int c0 = 0; c0 < limit && emitted < jhi; c0 += RS_NT * RS_PER) {
     int v[RS_PER];
     if (c0 == 0) {
 #pragma unroll
-      for (int k = 0; k < RS_PER; ++k) v[k] = k * NT + tid < limit ? v0[k] : -2;
+      for (int k = 0; k < RS_PER; ++k) v[k] = k * RS_NT + tid < limit ? v0[k] : -2;
     } else {
       load_slots(v, c0, limit);
     }
@@ -572,7 +571,7 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
 #pragma unroll
     for (int k = RS_PER - 1; k >= 0; --k) {
       const uint64_t m = __ballot(v[k] == -1);
-      if (m) first = c0 + k * NT + w * 64 + (int)__builtin_ctzll(m);
+      if (m) first = c0 + k * RS_NT + w * 64 + (int)__builtin_ctzll(m);
     }
     if (lane == 0) sh.wmin[w] = first;
     rs_barrier();
@@ -586,7 +585,7 @@ __device__ int resolve_rows(const SasFwdArgs& a, const int* tk, bool plan_ok, in
     int rank[RS_PER];
 #pragma unroll
     for (int k = 0; k < RS_PER; ++k) {
-      keep[k] = c0 + k * NT + tid < term && v[k] >= 0 && v[k] < thr;
+      keep[k] = c0 + k * RS_NT + tid < term && v[k] >= 0 && v[k] < thr;
       const uint64_t m = __ballot(keep[k]);
       rank[k] = __popcll(m & below);
       if (lane == 0) sh.cnt[k][w] = __popcll(m);
@@ -673,7 +672,7 @@ constexpr int RS_COPY = 8 * RS_NT;  // plan entries per copying workgroup
 template <bool INV>
 __global__ __launch_bounds__(RS_NT) void resolve_kernel(SasFwdArgs a, const int* __restrict__ plan,
                                                         SasResolveArgs r) {
-  __shared__ RsShared<RS_NT> sh;
+  __shared__ RsShared sh;
   // A plan built for other arguments is refused: every token resolves to no rows,
   // the attention kernel writes zeros and the combine kernel sets the status word.
   const bool plan_ok = plan_matches(plan, a);
@@ -693,7 +692,7 @@ __global__ __launch_bounds__(RS_NT) void resolve_kernel(SasFwdArgs a, const int*
   }
   const int* tk = plan + SAS_PLAN_HDR + (size_t)t * SAS_TOK_W;
   int nwin = 0;
-  const int n = resolve_rows<INV, RS_NT>(a, tk, plan_ok, t, 0, a.list_stride, sh, r, nwin);
+  const int n = resolve_rows<INV>(a, tk, plan_ok, t, 0, a.list_stride, sh, r, nwin);
   if (threadIdx.x == 0 && r.tok) r.tok[t] = make_int2(nwin, nwin < 0 ? 0 : n);
 }
 
