@@ -28,8 +28,8 @@
 // & 3), rope rows of 128 B with chunk c at c ^ ((r >> 1) & 7), as in the 32-key tile: the
 // b128 K reads (16 rows, one chunk) and the transposed V reads (4 rows x 4 chunks per 16
 // lanes) touch every bank once per 256 B.  A wave's 8 rope rows are one DMA (lane 8 k + j:
-// chunk j of row k, from per-lane addresses loaded a tile ahead) instead of one of 8
-// lanes per row.
+// chunk j of row k; the row addresses, in SGPRs a tile ahead, are moved into the lanes
+// before it) instead of one of 8 lanes per row.
 #include <hip/hip_runtime.h>
 
 #include "sas_common.h"

@@ -22,7 +22,7 @@
 //                     dO): one workgroup per work unit, the tile's gradient summed
 //                     over all heads in registers, then fp32 atomics into
 //                     pool-shaped buffers (one per element and tile).
-//   bwd_dsink_kernel  dsink[h] summed over tokens in a fixed order (one wave per
+//   bwd_dsink_kernel  dsink[h] summed over tokens in a fixed order (one workgroup per
 //                     head), so it is deterministic.
 //
 // MFMA 16x16x32 operand layouts (lane l, n = l & 15, g = l >> 4): A (16 x 32)
@@ -151,16 +151,26 @@ struct DqLds {
   __attribute__((aligned(16))) uint8_t tp[SPILL ? 4 * 2048 : 16];
 };
 
-// Ring of three tiles: tile i is computed while tile i + 1 arrives and tile i + 2's DMAs
-// (wave w: rows 8 w .. + 7, 8 latent and one rope instruction) are issued between the
-// S / dP chain's MFMAs; one barrier per tile.  What bounds it is the S / dP chain (36
-// k-steps, one LDS read and two dependent MFMAs each, on the SIMD's only wave: q, dO and
-// dq^T fill its registers).  Before, the next tile's rows went through registers and a
-// second barrier, the first tile was fetched after the query's rows, and the check for
-// infinities and NaNs took four instructions per value.  Measured, with the spill: 4 documents
-// of 608 .. 1,697 tokens, 128 heads, top-k 512, 1,390 -> 1,070 us; documents of 1,082
-// and 971 tokens, 64 heads, window only, d_qk 512, 232 -> 185 us (and since it computes D
-// too 1,170 and 210 us).
+// Ring of three tiles, one barrier per tile: tile i + 2's DMAs (wave w: rows 8 w .. + 7, 8
+// latent and one rope instruction) are issued between the MFMAs of tile i's S / dP chain.
+// They have that one tile's time to arrive, not two: the row addresses of tile i + 3 are
+// loaded behind them, vector memory completes in order, and the next iteration begins by
+// waiting for those addresses, so two of the three slots are in flight or in use.
+//
+// What bounds it: a workgroup reads its 64 heads' q, dO and out rows and writes their dq in
+// fp32, 352 KB (328 KB at d_qk 512), before and after its tiles and, one workgroup
+// per CU (125 KB of LDS, 380 registers), beside nothing else; at the rate of a large copy
+// that is 17.7 us (16.5) when every CU does it.  Window-only calls of 8,192 tokens whose
+// units have 1, 2, 4, 8, 16 and 32 tiles take 22.0, 22.8, 24.7, 31.0, 46.4 and 71.0 us per
+// workgroup at 128 heads with the spill (21.4, 22.9, 25.7, 28.5, 38.8, 58.5 without it) and
+// 18.5, 20.9, 24.2, 30.1, 42.7 and 61.4 us at 64 heads, d_qk 512: a long unit's tile is
+// 1.2 to 1.9 us (1.1 to 1.3), 0.7 of them MFMA (104 per wave, 1,664 cycles).
+//
+// Before, the next tile's rows went through registers and a second barrier, the first tile
+// was fetched after the query's rows, and the check for infinities and NaNs took four
+// instructions per value.  Measured, with the spill: 4 documents of 608 .. 1,697 tokens, 128
+// heads, top-k 512, 1,390 -> 1,070 us; documents of 1,082 and 971 tokens, 64 heads, window
+// only, d_qk 512, 232 -> 185 us (and since it computes D too 1,170 and 211 us).
 template <int DQK, int QT, bool SPILL>
 __device__ __forceinline__ void dq_unit(DqLds<DQK, SPILL>& sm, const int4 ur, int hg, const SasFwdArgs& a,
                                         const uint16_t* __restrict__ q, const uint16_t* __restrict__ dout,
@@ -338,7 +348,9 @@ __device__ __forceinline__ void dq_unit(DqLds<DQK, SPILL>& sm, const int4 ur, in
   for (int i = 0; i < ntiles; ++i) {
     const int rb = r0 + i * BW_TILE;
     // Tile i has landed: younger are tile i + 1's DMAs, an address load and, from the
-    // second tile on, the last tile's stores (in the first, the query's loads)
+    // second tile on, the last tile's stores (in the first, the query's loads).  (The wait
+    // for the addresses behind the barrier, which the compiler places, is the stricter one
+    // from the second tile on: all but those stores.)
     if (i == 0)
       __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
     else

@@ -192,7 +192,12 @@ bool fused_resolution(const sas_params_t* p, int target) {
 // tiles.  Where every unit starts at once nothing runs beside it, and the four-wave
 // kernel's wider gather and resolution win (32 sequences of 4k to 32k tokens, 64 heads,
 // top-k 512, a graph replay: 32.6 us against 35.2 us with two waves; 101 tokens of 16
-// heads, top-k 1024, an eager step with its plan: 125 against 147 us).
+// heads, top-k 1024, an eager step with its plan: 125 against 147 us).  Below 33 heads the
+// second wave's heads do not exist either, of two instead of four: forward calls of three
+// prompts of 2,000 tokens, top-k 512, d_qk 576, take 391 (16 heads), 408 (32), 409 (33) and
+// 463 us (64) against 641, 666, 668 and 709 with four waves; a window-only prompt of 8,192,
+// d_qk 512, 244 (8), 253 (16), 282 (32) and 342 (64) against 381, 393, 433 and 490; 300
+// tokens of one prompt 35 (16) and 39 (64) against 44 and 49.
 bool narrow_heads(const sas_params_t* p, int target) {
   return p->num_heads_q <= 64 && p->kv_dtype != SAS_DT_FP8E4M3 && !fused_resolution(p, target);
 }
