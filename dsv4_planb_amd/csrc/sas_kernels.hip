@@ -678,8 +678,8 @@ __global__ __launch_bounds__(RS_NT) void resolve_kernel(SasFwdArgs a, const int*
   const bool plan_ok = plan_matches(plan, a);
   const int t = (int)blockIdx.x - r.copies + r.t0;
   if ((int)blockIdx.x < r.copies) {
-    const int64_t n = SAS_PLAN_HDR + (int64_t)a.T * SAS_TOK_W +
-                      (int64_t)min(plan[PH_UNITS], a.unit_cap) * SAS_UNIT_W;
+    // (to the unit capacity, which a matching plan's buffer holds)
+    const int64_t n = SAS_PLAN_HDR + (int64_t)a.T * SAS_TOK_W + (int64_t)a.unit_cap * SAS_UNIT_W;
     const int64_t i0 = (int64_t)blockIdx.x * RS_COPY + threadIdx.x;
     if (!plan_ok) {
       if (i0 < SAS_PLAN_HDR) r.local[i0] = 0;
