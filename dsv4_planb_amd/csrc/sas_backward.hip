@@ -170,7 +170,7 @@ struct DqLds {
 // was fetched after the query's rows, and the check for infinities and NaNs took four
 // instructions per value.  Measured, with the spill: 4 documents of 608 .. 1,697 tokens, 128
 // heads, top-k 512, 1,390 -> 1,070 us; documents of 1,082 and 971 tokens, 64 heads, window
-// only, d_qk 512, 232 -> 185 us (and since it computes D too 1,170 and 211 us).
+// only, d_qk 512, 232 -> 185 us (and since it computes D too 1,175 and 217 us).
 template <int DQK, int QT, bool SPILL>
 __device__ __forceinline__ void dq_unit(DqLds<DQK, SPILL>& sm, const int4 ur, int hg, const SasFwdArgs& a,
                                         const uint16_t* __restrict__ q, const uint16_t* __restrict__ dout,

@@ -23,10 +23,10 @@
 // as the bound.
 //
 // Measured (the pools' gradient of packed training batches, before: the per-unit kernel):
-// 4 documents of 608 .. 1,697 tokens, 128 heads, top-k 512: 2,424 -> 569 us (and 300 us
+// 4 documents of 608 .. 1,697 tokens, 128 heads, top-k 512: 2,424 -> 565 us (and 300 us
 // for the spill in the dq kernel as it was then); documents of 1,082 and 971 tokens, 64
-// heads, window only, d_qk 512: 424 -> 106 us (and 50 us).
-// What bounds it now is memory: 3.2 GB read in 569 us (5.6 TB/s), of which 1.7
+// heads, window only, d_qk 512: 424 -> 107 us (and 50 us).
+// What bounds it now is memory: 3.2 GB read in 565 us (5.7 TB/s), of which 1.7
 // GB are first reads.  A operands loaded by every wave that uses them (64 loads of 16
 // rows per step, instead of 16 DMAs into the ring) doubled its time: a load of 16
 // 64-B rows occupies the vector memory pipe about 40 cycles.
